@@ -910,12 +910,16 @@ def main():
     h, nsph, phi = build_pack(L, n, args.radius, args.phi, args.seed, args.force)
     N = n ** 3
 
-    kernel = L.slb_step_kernel(h).decode()
+    # runs with walls at rest take two steps per pass over the populations
+    # (k_step2), one read and one write for both, unless the environment
+    # names a single-step kernel
+    pairs = os.environ.get("SLB_STEP2", "1") != "0" and "SLB_STEP_LDS" not in os.environ
+    kernel = "k_step2" if pairs else L.slb_step_kernel(h).decode()
     L.slb_run(h, args.warmup)
     ms = L.slb_time_steps(h, args.steps)
     ms_per_step = ms / args.steps
     mlups = N * args.steps / (ms * 1e-3) / 1e6
-    bytes_per_lup = 2 * 15 * (4 if args.precision == 32 else 8)
+    bytes_per_lup = (1 if pairs else 2) * 15 * (4 if args.precision == 32 else 8)
     achieved = bytes_per_lup * N / (ms_per_step * 1e-3) / 1e9
     log(f"gpu: {ms_per_step * 1e3:.1f} us/step, {mlups:.1f} MLUPS, {achieved:.0f} GB/s "
         f"algorithmic ({bytes_per_lup} B/LUP)")
@@ -958,7 +962,8 @@ def main():
             "frac": round(achieved / PEAK_HBM_GBS, 4),
             "traffic": traffic_bytes(n, args.precision),
             # the kernel the library launches for this lattice's steps
-            "kernel": kernel + {"k_step_lds": " (fused pull step, k pulls staged in LDS)",
+            "kernel": kernel + {"k_step2": " (two fused pull steps per pass)",
+                                "k_step_lds": " (fused pull step, k pulls staged in LDS)",
                                 "k_step_ldsr": " (fused pull step, k pulls staged in LDS, "
                                                "whole rows per block)",
                                 "k_step": " (fused pull step)"}.get(kernel, ""),

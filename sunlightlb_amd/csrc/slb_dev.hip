@@ -37,6 +37,7 @@
 #include "slb_dev.h"
 
 #include "slb_kern.h"
+#include "slb_step2.h"
 
 /* ---------------------------------------------------------------------- */
 /* Fused step kernel.                                                      */
@@ -1396,6 +1397,8 @@ struct slbd_lattice {
   int sweep_nt_mid;         /* two-step sweep: non-temporal window stores */
   int step_lds;             /* step with the k pulls staged in LDS (k_step_lds) */
   int ldsr_rpb, ldsr_bs;    /* k_step_ldsr: rows per block, threads per block (0: off) */
+  int pairs, pair_nt;       /* runs take their steps two at a time (k_step2); its store hint */
+  Step2Plan plan2;
   void *mom[2];             /* moment storage of a run (k_step_mom), or NULL */
   void *sph_buf;            /* sphere images of a pack being placed (grow-only) */
   size_t sph_cap;
@@ -1461,6 +1464,26 @@ extern "C" const char *slbd_arch(void) {
   return name;
 }
 
+/* Whether runs with walls at rest take their steps two at a time (k_step2):
+ * always, since it is the faster one on every shape measured
+ * (slb_step2.hip), unless SLB_STEP2=0
+ * or the environment names a single-step kernel or 64-bit indices.  Lattices
+ * beyond 32-bit population indices need planes of whole population tiles.
+ * Stores are non-temporal except where both buffers fit the 256 MB last-level
+ * cache and exceed the L2s by far, and the next pass reads them there: nt /
+ * plain us per FP32 step at 96^3 (106 MB) 15.8/12.6, 128^3 (252 MB)
+ * 31.9/30.4, 160^3 (491 MB) 58.8/61.5, 64^3 (31 MB) 6.05/6.31. */
+static void pair_policy(slbd_lattice *L) {
+  const long np = 15 * pop_nodes(L->N), ts = (long)tsize(L->prec);
+  const char *e = getenv("SLB_STEP2");
+  const bool small = np <= 0x7fffffffL;
+  L->pairs = !(e && atoi(e) == 0) && !getenv("SLB_STEP_LDS") && L->idx32 == (int)small &&
+             (small || (L->G.plane % POP_TILE == 0 && 15L * L->G.plane * ts < (1L << 32))) &&
+             slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2);
+  const double both = 30.0 * (double)L->N * (double)ts;
+  L->pair_nt = L->G.nt_store && !(both > 64e6 && both <= 256e6);
+}
+
 /* The step kernel of a lattice, from its shape and precision (made again
  * when the precision changes).  k_step_lds needs whole rows per 512-thread
  * block. */
@@ -1501,6 +1524,7 @@ static void step_kernel_policy(slbd_lattice *L) {
       }
     }
   }
+  pair_policy(L);
 }
 
 extern "C" slbd_lattice *slbd_create(int esi, int esj, int esk, int prec) {
@@ -2249,6 +2273,13 @@ extern "C" void slbd_step(slbd_lattice *L, const slbd_params *P, int nsteps, int
       else sweep2<double>(L, A, P->moving != 0, bf, sw);
     }
   }
+  if (L->pairs && sw == 0 && !force && !P->moving)
+    for (; s + 2 <= nsteps; s += 2) {
+      const Step2Args a = {L->pops[L->cur], L->pops[L->cur ^ 1], L->flags, L->bx, L->by, L->bz,
+                           L->pair_nt != 0, bf, L->plan2};
+      slbd_step2_launch(&a, A, L->G, L->prec, L->stream);
+      L->cur ^= 1;
+    }
   for (; s < nsteps; s++) {
     void *src = L->pops[L->cur], *dst = L->pops[L->cur ^ 1];
     if (L->prec == 32)

@@ -1,0 +1,61 @@
+"""Runs with walls at rest take their steps two at a time (k_step2), single
+lbstep calls and moving walls do not.
+Populations after runs against the same number of lbstep calls, bit for bit
+(one function holds the collision of both kernels, so the tolerance is zero),
+at the edges of its tiles: k tiles with a remainder and rows of one node,
+j and i remainders, planes that are and are not whole population tiles,
+lattices of one plane, odd step counts."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def build(dims, prec, moving, stokes, skip, bf):
+    import sunlightlb_amd as s
+    lat = s.Lattice(*dims, precision=prec)
+    L, h = lat.L, lat.h
+    lat.s.tau, lat.s.stokes_flow, lat.s.skip_solid, lat.s.objects_moving = 0.7, stokes, skip, moving
+    rng = np.random.default_rng(sum(dims))
+    for q in range(max(3, lat.N // 4000)):
+        sph = L.insertsph(h, float(rng.uniform(0.8, 4.0)), *[float(rng.uniform(-1.0, n)) for n in dims])
+        if sph:
+            sph.contents.velx, sph.contents.vely = 0.01, -0.004 * (q % 3)
+            sph.contents.velz, sph.contents.angz = 0.006, 0.002
+    if moving:
+        L.vspread(h)
+    L.zerobf(h)
+    if bf == 2:
+        lat.sync()
+        solid = lat.solid()
+        for nm, sc in (("bx", 2e-4), ("by", 5e-5), ("bz", 1e-4)):
+            s.view(getattr(lat.s, nm), lat.N)[:] = np.where(solid, 0.0, sc * (1 + rng.random(lat.N)))
+        L.slb_sync_device(h)
+    elif bf == 1:
+        L.addbf(h, 1e-4, 0.0, 2e-5)
+    lat.set_pops(1e-3 * rng.standard_normal(lat.N * 15))
+    return lat
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("dims,moving,stokes,skip,bf", [
+    ((9, 32, 64), 1, 0, 1, 2),        # whole tiles per plane
+    ((7, 16, 256), 0, 1, 0, 1),       # more than one k tile
+    ((5, 8, 512), 1, 1, 0, 0),
+    ((13, 23, 75), 0, 0, 0, 2),       # remainders in j and k
+    ((4, 11, 331), 1, 0, 0, 1),       # k tiles of unequal width
+    ((70, 5, 9), 0, 1, 1, 1),         # many planes
+    ((1, 1, 7), 1, 0, 0, 1), ((2, 2, 2), 0, 0, 0, 1), ((3, 2, 1), 1, 1, 0, 2), ((2, 1024, 1), 0, 1, 0, 1),
+    ((96, 96, 96), 0, 1, 0, 1),       # plain stores (FP32: both buffers fit the cache)
+])
+def test_run_is_single_steps(prec, dims, moving, stokes, skip, bf):
+    print(f"pairs: {dims} prec {prec}", flush=True)
+    ref, got = (build(dims, prec, moving, stokes, skip, bf) for _ in range(2))
+    for n in (2, 7):
+        for _ in range(n):
+            ref.L.lbstep(ref.h)
+        got.L.slb_run(got.h, n)
+        assert np.array_equal(ref.pops(), got.pops())
+    assert got.s.step == 9
+    ref.free()
+    got.free()
