@@ -339,9 +339,8 @@ k_conv_wgrad(const uint16_t *__restrict__ X, int Cin, const uint16_t *__restrict
 
 /* ---------------------------------------------------------------------- */
 /* Weight gradient as a GEMM over the node-blocked layout                    */
-/*   Xb[((n >> 3) * C + c) * 8 + (n & 7)]                                     */
-/* (8 consecutive nodes of one channel in 16 bytes, x-rows of a multiple of  */
-/* 8 nodes).  Block (group range, tap t): M = Cout, N = Cin, K = nodes; the   */
+/*   Xb[((row * gW + x / 8) * C + c) * 8 + x % 8],  gW = ceil(Wd / 8)         */
+/* (8 consecutive nodes of an x-row of one channel in 16 bytes).  Block (group range, tap t): M = Cout, N = Cin, K = nodes; the   */
 /* 4 waves take interleaved K-steps of 32 nodes (4 groups) and are reduced in */
 /* LDS; partial sums per block go to part[t][block][co][ci] and are added in  */
 /* a fixed order by k_wgrad_reduce (deterministic).  The tap's x shift of one */
@@ -359,9 +358,36 @@ __global__ void k_block(const uint16_t *__restrict__ X, int C, uint16_t *__restr
   *(uint4 *)(Xb + e * 8) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+/* The same for x-rows that are no multiple of 8 nodes: the row's last group
+ * is filled up with zeros, and with wrap its first free place with the row's
+ * node 0, the periodic neighbour of the last node. */
+__global__ void k_block_pad(const uint16_t *__restrict__ X, int C, uint16_t *__restrict__ Xb,
+                            long rows, int Wd, int wrap) {
+  const int gW = (Wd + 7) >> 3;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= rows * gW * C) return;
+  const long g = e / C, row = g / gW;
+  const int c = (int)(e - g * C), x0 = (int)(g - row * gW) * 8;
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    uint32_t h[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      const int x = x0 + 2 * k + q;
+      const bool in = x < Wd || (wrap && x == Wd);
+      h[q] = in ? X[(row * Wd + (x < Wd ? x : 0)) * C + c] : 0;
+    }
+    w[k] = h[0] | (h[1] << 16);
+  }
+  *(uint4 *)(Xb + e * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+}
 
-
-template <int MT, int NT, int TX>
+/* PAD: x-rows that are no multiple of 8 nodes, from k_block_pad.  The zeros
+ * of the output gradient take the row's last places out of every sum; the
+ * place after the last node holds node 0 (dx = +1), and node 0's left
+ * neighbour is taken from the row's last node (dx = -1). */
+template <int MT, int NT, int TX, bool PAD>
 __global__ void __launch_bounds__(256)
 k_wgrad_b(const uint16_t *__restrict__ Xb, const uint16_t *__restrict__ Db,
           float *__restrict__ part, int gpb, NGeom G) {
@@ -375,8 +401,9 @@ k_wgrad_b(const uint16_t *__restrict__ Xb, const uint16_t *__restrict__ Db,
   const int dz = TX == 3 ? tq / 3 - 1 : tq / 9 - 1;
   const int dy = TX == 3 ? tq % 3 - 1 : (tq / 3) % 3 - 1;
   const int dx1 = TX == 3 ? 0 : tq % 3 - 1;   /* the single dx of TX = 1 */
-  const int gW = G.Wd >> 3;
-  const long ngr = (long)G.N >> 3;
+  const int gW = PAD ? (G.Wd + 7) >> 3 : G.Wd >> 3;
+  const int tail = (G.Wd - 1) & 7;                     /* place of a row's last node */
+  const long ngr = PAD ? (long)G.D * G.H * gW : (long)G.N >> 3;
   const long gb = (long)blockIdx.x * gpb;
   const long ge = min(ngr, gb + gpb);
   f32x4 acc[TX][MT][NT];
@@ -427,7 +454,12 @@ k_wgrad_b(const uint16_t *__restrict__ Xb, const uint16_t *__restrict__ Db,
           v.w = (v0.w >> 16) | (vp.x << 16);
         } else {
           /* nodes x0-1 .. x0+6: element 7 of vm, elements 0..6 of v0 */
-          v.x = (vm.w >> 16) | (v0.x << 16);
+          uint32_t left = vm.w >> 16;
+          if (PAD && xg == 0) {
+            const uint32_t wd = tail < 2 ? vm.x : tail < 4 ? vm.y : tail < 6 ? vm.z : vm.w;
+            left = (tail & 1) ? wd >> 16 : wd & 0xffffu;
+          }
+          v.x = left | (v0.x << 16);
           v.y = (v0.x >> 16) | (v0.y << 16);
           v.z = (v0.y >> 16) | (v0.z << 16);
           v.w = (v0.z >> 16) | (v0.w << 16);
@@ -1094,8 +1126,8 @@ static void *wg_workspace(size_t bytes) {
   return wg_ws;
 }
 
-/* the original per-tap LDS-staged kernel: any extents (used when the
- * x-rows are not a multiple of 8 nodes) */
+/* the per-tap LDS-staged kernel with atomics: the channel counts that the
+ * blocked one does not cover (48) */
 static void wgrad_staged(const uint16_t *X, int cin, const uint16_t *dY, int cout, float *dW,
                          const NGeom &G) {
   const int Kp = slbn_kpad(cin);
@@ -1124,8 +1156,8 @@ extern "C" int slbn_wgrad_lds16_ok(int cin, int cout, int D, int H, int Wd) {
 }
 
 extern "C" int slbn_wgrad_blocked_ok(int cin, int cout, int D, int H, int Wd) {
-  (void)D; (void)H;
-  return Wd % 8 == 0 && (cin == 16 || cin == 32 || cin == 64) &&
+  (void)D; (void)H; (void)Wd;
+  return (cin == 16 || cin == 32 || cin == 64) &&
          (cout == 16 || cout == 32 || cout == 64);
 }
 
@@ -1156,7 +1188,12 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
     LAUNCHCHECK();
     return;
   }
-  const long ngr = (long)G.N >> 3;
+  /* rows of any length in groups of 8 nodes; the padded groups cost at most
+   * 8/9 of the work at rows of 9 nodes and replace 27 launches of the per-tap
+   * kernel (96 x 80 x 72 network, its level of 36-node rows: 27 x 63 us
+   * against 34 us) */
+  const bool pad = Wd % 8 != 0;
+  const long ngr = (long)D * H * ((Wd + 7) >> 3);
   /* enough blocks per tap to fill the chip with 27 taps, each block a
    * contiguous group range in steps of 16 groups */
   const int mt = cout / 16, nt = cin / 16;
@@ -1168,21 +1205,36 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
   if (nb < 1) nb = 1;
   int gpb = (int)(((ngr + nb - 1) / nb + 15) / 16 * 16);
   nb = (ngr + gpb - 1) / gpb;
-  const size_t xb = (size_t)G.N * cin * 2, db = (size_t)G.N * cout * 2;
+  const size_t xb = (size_t)ngr * 8 * cin * 2, db = (size_t)ngr * 8 * cout * 2;
   const size_t pb = (size_t)27 * nb * cout * cin * 4;
   char *ws = (char *)wg_workspace(xb + db + pb);
   uint16_t *Xb = (uint16_t *)ws, *Db = (uint16_t *)(ws + xb);
   float *part = (float *)(ws + xb + db);
-  hipLaunchKernelGGL(k_block, dim3(blocks_for(ngr * cin, 256)), dim3(256), 0, nn_stream, X, cin,
-                     Xb, (long)G.N);
+  const long rows = (long)D * H;
+  if (pad)
+    hipLaunchKernelGGL(k_block_pad, dim3(blocks_for(ngr * cin, 256)), dim3(256), 0, nn_stream, X,
+                       cin, Xb, rows, Wd, 1);
+  else
+    hipLaunchKernelGGL(k_block, dim3(blocks_for(ngr * cin, 256)), dim3(256), 0, nn_stream, X, cin,
+                       Xb, (long)G.N);
   LAUNCHCHECK();
-  hipLaunchKernelGGL(k_block, dim3(blocks_for(ngr * cout, 256)), dim3(256), 0, nn_stream, dY, cout,
-                     Db, (long)G.N);
+  if (pad)
+    hipLaunchKernelGGL(k_block_pad, dim3(blocks_for(ngr * cout, 256)), dim3(256), 0, nn_stream, dY,
+                       cout, Db, rows, Wd, 0);
+  else
+    hipLaunchKernelGGL(k_block, dim3(blocks_for(ngr * cout, 256)), dim3(256), 0, nn_stream, dY,
+                       cout, Db, (long)G.N);
   LAUNCHCHECK();
   const dim3 grid((unsigned)nb, 27 / tx);
-#define SLBN_WGB(MT, NT, TX)                                                             \
-  hipLaunchKernelGGL((k_wgrad_b<MT, NT, TX>), grid, dim3(256), 0, nn_stream, Xb, Db, part, \
-                     gpb, G)
+#define SLBN_WGB(MT, NT, TX)                                                              \
+  do {                                                                                    \
+    if (pad)                                                                              \
+      hipLaunchKernelGGL((k_wgrad_b<MT, NT, TX, true>), grid, dim3(256), 0, nn_stream, Xb, \
+                         Db, part, gpb, G);                                               \
+    else                                                                                  \
+      hipLaunchKernelGGL((k_wgrad_b<MT, NT, TX, false>), grid, dim3(256), 0, nn_stream, Xb, \
+                         Db, part, gpb, G);                                               \
+  } while (0)
   if (mt == 1 && nt == 1) SLBN_WGB(1, 1, 3);
   else if (mt == 1 && nt == 2) SLBN_WGB(1, 2, 3);
   else if (mt == 2 && nt == 1) SLBN_WGB(2, 1, 3);
@@ -1364,8 +1416,38 @@ __global__ void k_expand(const uint16_t *__restrict__ S, int Cs, uint16_t *__res
   X[e] = (c < Cs) ? S[n * Cs + c] : (uint16_t)0;
 }
 
+/* The same with 8 channels per thread and 16-byte stores (loads too where Cs
+ * is a multiple of 8): one 2-byte value per thread took 73 us for 16 to 16
+ * channels at 128^3 (1.8 TB/s). */
+__global__ void __launch_bounds__(256)
+k_expand8(const uint16_t *__restrict__ S, int Cs, uint16_t *__restrict__ X, int C, int wide,
+          long N) {
+  const int G8 = C >> 3;
+  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= N * G8) return;
+  const long n = e / G8;
+  const int c0 = (int)(e - n * G8) * 8;
+  u32x4 v = (u32x4){0u, 0u, 0u, 0u};
+  if (wide) {
+    if (c0 < Cs) v = *(const u32x4 *)(S + n * Cs + c0);
+  } else {
+    uint32_t h[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) h[q] = c0 + q < Cs ? S[n * Cs + c0 + q] : 0u;
+    v = (u32x4){h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+  }
+  ((u32x4 *)X)[e] = v;
+}
+
 extern "C" void slbn_expand(const uint16_t *S, int Cs, uint16_t *X, int C, long N) {
-  hipLaunchKernelGGL(k_expand, dim3(blocks_for(N * C, 256)), dim3(256), 0, nn_stream, S, Cs, X, C, N);
+  if (C % 8 == 0 && ((uintptr_t)X & 15) == 0) {
+    const int wide = Cs % 8 == 0 && ((uintptr_t)S & 15) == 0;
+    hipLaunchKernelGGL(k_expand8, dim3(blocks_for(N * (C / 8), 256)), dim3(256), 0, nn_stream, S, Cs,
+                       X, C, wide, N);
+  } else {
+    hipLaunchKernelGGL(k_expand, dim3(blocks_for(N * C, 256)), dim3(256), 0, nn_stream, S, Cs, X, C,
+                       N);
+  }
   LAUNCHCHECK();
 }
 

@@ -1,0 +1,97 @@
+"""The warm-start network's weight gradient on x-rows of any length, its
+input expansion, and the lattice hooks' features and moments, at the edges
+of their groups and blocks.  Bars as in test_gpu_warm.py: FP32 weight
+gradients within 1e-5 of the oracle relative to the largest value, features
+and copies bit-exact."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from oracle import nn as onn
+from test_gpu_warm import Dev, bf_random, lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (64, 32), (64, 64)])
+@pytest.mark.parametrize("shape", [(3, 4, 1), (4, 3, 2), (2, 5, 7), (3, 3, 9), (5, 4, 12), (4, 2, 23),
+                                   (2, 3, 36), (6, 5, 18), (2, 2, 141)])
+def test_weight_gradient_on_ragged_rows(shape, cin, cout):
+    L = lib()
+    print(f"ragged wgrad {shape} {cin}->{cout}", flush=True)
+    assert L.slbn_wgrad_blocked_ok(cin, cout, *shape)
+    rng = np.random.default_rng(sum(shape) + cin + cout)
+    xb, x = bf_random(rng, shape + (cin,))
+    gb, g = bf_random(rng, shape + (cout,))
+    kp = onn.kpad(cin)
+    dX, dG, dW = Dev(host=xb), Dev(host=gb), Dev(cout * kp * 4)
+    L.slbn_conv_wgrad(dX.p, cin, dG.p, cout, dW.p, *shape)
+    L.slbn_sync()
+    got = dW.get(np.float32, (cout, kp)).astype(np.float64)
+    for d in (dX, dG, dW):
+        d.free()
+    ref = onn.conv3d_bwd_weight(x, g).reshape(cout, 27 * cin)
+    assert np.all(got[:, 27 * cin:] == 0.0)
+    assert np.abs(got[:, :27 * cin] - ref).max() < 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("cs,c", [(2, 16), (16, 16), (8, 16), (10, 16), (3, 12), (24, 8)])
+def test_expand(cs, c):
+    L = lib()
+    n = 773
+    s = np.random.default_rng(cs + c).integers(0, 1 << 16, (n, cs)).astype(np.uint16)
+    dS, dX = Dev(host=s), Dev(n * c * 2)
+    L.slbn_expand(dS.p, cs, dX.p, c, n)
+    L.slbn_sync()
+    want = np.zeros((n, c), np.uint16)
+    want[:, :min(cs, c)] = s[:, :min(cs, c)]
+    assert np.array_equal(dX.get(np.uint16, (n, c)), want)
+    dS.free()
+    dX.free()
+
+
+@pytest.mark.parametrize("dims", [(5, 7, 3), (2, 3, 1030), (17, 4, 33), (1, 1, 6)])
+def test_features_at_odd_extents(dims):
+    """Seeds as coordinates (extents up to 1024) and as node indices."""
+    import sunlightlb_amd as s
+    lat = s.Lattice(*dims, precision=64)
+    solid = np.random.default_rng(sum(dims)).random(dims) < 0.1
+    solid.reshape(-1)[0] = True
+    m = np.ascontiguousarray(solid.astype(np.uint8).reshape(-1))
+    lat.L.slb_insert_map(lat.h, m.ctypes.data_as(C.c_void_p))
+    f, ell_ref = onn.features(solid)
+    for ch in (2, 8, 16, 3):
+        dF = Dev(lat.N * ch * 2)
+        ell = lat.L.slb_warm_features(lat.h, dF.p, ch)
+        got = dF.get(np.uint16, dims + (ch,))
+        dF.free()
+        assert abs(ell - ell_ref) < 1e-12 * ell_ref
+        want = np.zeros(dims + (ch,), np.uint16)
+        want[..., :2] = onn.bf16_bits(f)
+        assert np.array_equal(got, want)
+    lat.free()
+
+
+@pytest.mark.parametrize("dims", [(3, 5, 7), (4, 8, 8), (5, 9, 23)])
+def test_moments_of_any_channel_count(dims):
+    """The moments' first channels are the same whatever the channel count."""
+    import sunlightlb_amd as s
+    lat = s.Lattice(*dims, precision=64)
+    lat.L.insertsph(lat.h, 1.5, 1.0, 2.0, 3.0)
+    lat.s.dpdx = 1e-3
+    lat.set_pops(1e-3 * np.random.default_rng(3).standard_normal(lat.N * 15))
+    out = {}
+    for ch in (10, 16, 4, 13, 300):
+        d = Dev((lat.N * ch + 64) * 4)
+        lat.L.slb_warm_moments(lat.h, d.p, ch, 1.0)
+        a = d.get(np.float32, (lat.N * ch + 64,))
+        d.free()
+        assert np.all(a[lat.N * ch:] == 0.0)
+        out[ch] = a[:lat.N * ch].reshape(lat.N, ch)
+        assert np.all(out[ch][:, 10:] == 0.0)
+    for ch in (16, 4, 13, 300):
+        q = min(10, ch)
+        assert np.array_equal(out[ch][:, :q], out[10][:, :q])
+    assert np.abs(out[10]).max() > 0.0
+    lat.free()
