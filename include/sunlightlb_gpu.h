@@ -148,7 +148,9 @@ void slb_mp_sums(MPSys mp, double out[6]);
  * more (SLB_MP_WEIGHTS=n sets the minimum, 0 never) computes each node's
  * link factors from the frozen flow once and reuses them: the tracer a
  * partially adsorbing node keeps is then (sum of its link factors) x P
- * instead of the sum of the products, a rounding-level difference. */
+ * instead of the sum of the products, a rounding-level difference.  Large
+ * lattices take two steps per pass over the factors (SLB_MP_STEP2=0 never, 1
+ * always), with the same results. */
 void slb_mp_run(MPSys mp, int nsteps);
 
 /* Time nsteps MP steps on the device between HIP events (the state

@@ -38,6 +38,7 @@
 
 #include "slb_kern.h"
 #include "slb_step2.h"
+#include "slb_mpk.h"
 
 /* ---------------------------------------------------------------------- */
 /* Fused step kernel.                                                      */
@@ -966,7 +967,8 @@ k_mprho(const T *__restrict__ a, const uint16_t *__restrict__ flags, double rho0
 
 /* MP flags: bit l (0..14) = node x - c_l is fluid; bit 16+l (1..14) = node
  * s = x - c_l is a solid with boundary link l that reflects (mask bit l-1
- * set, adsorption bit 0x4000 clear). */
+ * set, adsorption bit 0x4000 clear); on a solid x bit 15 = it adsorbs (mask bit
+ * 0x4000), bit 16 = it is a boundary node (mask not 0). */
 __global__ void __launch_bounds__(256)
 k_mpflags(const int32_t *__restrict__ objidx, const int32_t *__restrict__ mask,
           uint32_t *__restrict__ mpf, Geom G) {
@@ -977,7 +979,8 @@ k_mpflags(const int32_t *__restrict__ objidx, const int32_t *__restrict__ mask,
   const AxisOff oi = axis_off(i, G.esi, G.plane);
   const AxisOff oj = axis_off(j, G.esj, G.esk);
   const AxisOff ok = axis_off(k, G.esk, 1);
-  uint32_t f = (objidx[x] < 0) ? 1u : 0u;
+  const int mx = mask[x];
+  uint32_t f = (objidx[x] < 0) ? 1u : ((mx & 0x4000) ? 1u << 15 : 0u) | (mx != 0 ? 1u << 16 : 0u);
   Links<1, 15>::run([&](auto LL) {
     constexpr int l = decltype(LL)::value;
     const long s = x + nb_off<l, -1>(oi, oj, ok);
@@ -990,11 +993,6 @@ k_mpflags(const int32_t *__restrict__ objidx, const int32_t *__restrict__ mask,
   });
   mpf[x] = f;
 }
-
-struct MPArgs {
-  double rho0, alpha, pads;
-  int axis;
-};
 
 /* MP fields live in node records of W = 2 (P, 1/rho) or W = 4 (P, m1, m2,
  * 1/rho) values, so that the gather below reads one vector per incoming link
@@ -1015,9 +1013,8 @@ template <typename T, int NMOM, bool MOVING, typename I>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(1, sizeof(T) == 8 ? 4 : 8)))
 k_mpstep(const T *__restrict__ a, const T *__restrict__ qin, T *__restrict__ qout,
-         const uint32_t *__restrict__ mpf, const int32_t *__restrict__ mask,
-         const int32_t *__restrict__ objidx, const double *__restrict__ tab,
-         Geom G, MPArgs A) {
+         const uint32_t *__restrict__ mpf, const int32_t *__restrict__ objidx,
+         const double *__restrict__ tab, Geom G, MPArgs A) {
   constexpr int W = NMOM > 1 ? 4 : 2;
   typedef T V __attribute__((ext_vector_type(W)));
   const V *__restrict__ Q = (const V *)qin;
@@ -1107,10 +1104,7 @@ k_mpstep(const T *__restrict__ a, const T *__restrict__ qin, T *__restrict__ qou
     o[0] = np;
     if (NMOM > 1) { o[1] = n1; o[2] = n2; }
   } else {
-    const int m = mask[x];
-    T frac = T(0);
-    if (m & 0x4000) frac = T(1);
-    else if (m != 0 && A.pads > 0.0) frac = T(A.pads);
+    const T frac = mp_kept<T>(f, A);
     if (frac != T(0)) {
       o[0] = qx[0] + frac * np;
       if (NMOM > 1) { o[1] = qx[1] + frac * n1; o[2] = qx[2] + frac * n2; }
@@ -1136,19 +1130,6 @@ k_mpstep(const T *__restrict__ a, const T *__restrict__ qin, T *__restrict__ qou
  * and gathers only the records.  The one difference in arithmetic: the
  * kept own tracer is (sum of the own factors) x P rather than the sum of
  * the products. */
-/* weights in tiles of 1024 nodes: runs of 1024 four-value vectors (weights
- * 0-3, 4-7, 8-11) and one of 1024 three-value vectors (12-14), so a wave's
- * load of one run is contiguous */
-template <typename I>
-__device__ __forceinline__ I wt_idx(int c, I x) {
-  const I tile = (x >> POP_SHIFT) * I(15 * POP_TILE), n = x & I(POP_TILE - 1);
-  return c < 3 ? tile + (I(c) * I(POP_TILE) + n) * I(4) : tile + I(12 * POP_TILE) + n * I(3);
-}
-template <typename T>
-struct __attribute__((aligned(sizeof(T)))) Wt3 {
-  T a, b, c;
-};
-
 template <typename T, bool MOVING, typename I>
 __global__ void __launch_bounds__(256)
 k_mpweights(const T *__restrict__ a, const T *__restrict__ qin, T *__restrict__ wt,
@@ -1202,13 +1183,6 @@ k_mpweights(const T *__restrict__ a, const T *__restrict__ qin, T *__restrict__ 
   *(Wt3<T> *)(wt + wt_idx<I>(3, x)) = Wt3<T>{w[12], w[13], w[14]};
 }
 
-/* Compact node records of a run on link factors: {P} or {P, m1, m2} without
- * the 1/rho slot, which only the factors use (12 bytes per node FP32 with
- * moments instead of 16). */
-template <typename T, int NM> struct CRec;
-template <typename T> struct __attribute__((aligned(sizeof(T)))) CRec<T, 3> { T p, m1, m2; };
-template <typename T> struct __attribute__((aligned(sizeof(T)))) CRec<T, 1> { T p; };
-
 template <typename T, int NM>
 __global__ void k_rec_pack(const T *__restrict__ q, int W, CRec<T, NM> *__restrict__ c, long N) {
   const long x = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1233,8 +1207,8 @@ template <typename T, int NMOM, typename I>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(1, sizeof(T) == 8 ? 4 : 8)))
 k_mpstep_w(const T *__restrict__ wt, const CRec<T, NMOM> *__restrict__ Q,
-           CRec<T, NMOM> *__restrict__ qout, const uint32_t *__restrict__ mpf,
-           const int32_t *__restrict__ mask, Geom G, MPArgs A) {
+           CRec<T, NMOM> *__restrict__ qout, const uint32_t *__restrict__ mpf, Geom G,
+           MPArgs A) {
   typedef T V4 __attribute__((ext_vector_type(4)));
   typedef CRec<T, NMOM> R;
   Geom Gb = G;
@@ -1291,10 +1265,7 @@ k_mpstep_w(const T *__restrict__ wt, const CRec<T, NMOM> *__restrict__ Q,
     o.p = np;
     if constexpr (NMOM > 1) { o.m1 = n1; o.m2 = n2; }
   } else {
-    const int m = mask[x];
-    T frac = T(0);
-    if (m & 0x4000) frac = T(1);
-    else if (m != 0 && A.pads > 0.0) frac = T(A.pads);
+    const T frac = mp_kept<T>(f, A);
     if (frac != T(0)) {
       o.p = qx.p + frac * np;
       if constexpr (NMOM > 1) { o.m1 = qx.m1 + frac * n1; o.m2 = qx.m2 + frac * n2; }
@@ -1411,6 +1382,8 @@ struct slbd_mp {
   long rho_version;  /* lattice density version the 1/rho slots hold */
   void *wt;        /* gather weights of the current run (15 per node, tiled), or NULL */
   void *cq[2];     /* compact records of a run on the weights, or NULL */
+  MP2Plan plan2;   /* tiles of two steps per pass (made at the first run) */
+  int planned;
 };
 
 static size_t tsize(int prec) { return prec == 32 ? sizeof(float) : sizeof(double); }
@@ -2668,6 +2641,25 @@ static int mp_weights_min(void) {
   return e ? atoi(e) : 32;
 }
 
+/* Whether the steps on link factors go two per pass (k_mpstep2): where the
+ * factors are larger than the eight 4 MB L2s together; smaller ones are read
+ * from there at every step, and the pair only adds its rims and barriers.
+ * Single / paired, us per FP32 step with moments: 64^3 (16 MB of factors)
+ * 4.7/5.9, 80^3 (31 MB) 8.8/9.7, 100 x 90 x 70 (38 MB) 12.5/10.8, 128^3
+ * 26.5/19.7, 256^3 322/153; FP64: 64^3 (31 MB) 10.3/11.4, 120 x 61 x 45 (40 MB)
+ * 12.9/11.3, 128^3 78.7/44.2.  SLB_MP_STEP2=0 never, =1 wherever a tile fits
+ * (read per call). */
+static bool mp_pairs(const slbd_lattice *L, slbd_mp *M) {
+  const char *e = getenv("SLB_MP_STEP2");
+  const bool large = 15.0 * (double)L->N * (double)tsize(L->prec) >= 36e6;
+  if (!L->idx32 || !(e ? atoi(e) != 0 : large)) return false;
+  if (!M->planned) {
+    M->planned = 1;
+    slbd_mp2_plan(L->esi, L->esj, L->esk, L->prec, M->nmom, &M->plan2);
+  }
+  return M->plan2.ci > 0;
+}
+
 template <typename T, int NMOM, bool MOVING>
 static void launch_mp_w(slbd_lattice *L, slbd_mp *M, const MPArgs &A, int nsteps) {
   if (!M->wt) M->wt = dalloc((size_t)pop_nodes(L->N) * 15 * sizeof(T));
@@ -2688,16 +2680,23 @@ static void launch_mp_w(slbd_lattice *L, slbd_mp *M, const MPArgs &A, int nsteps
   hipLaunchKernelGGL((k_rec_pack<T, NMOM>), lin_grid(L->N), dim3(256), 0, L->stream,
                      (const T *)M->q[M->cur], M->W, (R *)M->cq[0], L->N);
   LAUNCHCHECK();
-  int c = 0;
-  for (int s = 0; s < nsteps; s++) {
+  int c = 0, s = 0;
+  if (mp_pairs(L, M)) {
+    for (; s + 2 <= nsteps; s += 2) {
+      slbd_mp2_launch(M->wt, M->cq[c], M->cq[c ^ 1], L->mpf, L->prec, NMOM, L->G, A, M->plan2,
+                      L->stream);
+      c ^= 1;
+    }
+  }
+  for (; s < nsteps; s++) {
     if (L->idx32)
       hipLaunchKernelGGL((k_mpstep_w<T, NMOM, int>), plane_grid(L), dim3(256), 0,
                          L->stream, (const T *)M->wt, (const R *)M->cq[c], (R *)M->cq[c ^ 1],
-                         L->mpf, L->mask, L->G, A);
+                         L->mpf, L->G, A);
     else
       hipLaunchKernelGGL((k_mpstep_w<T, NMOM, long>), plane_grid(L), dim3(256), 0,
                          L->stream, (const T *)M->wt, (const R *)M->cq[c], (R *)M->cq[c ^ 1],
-                         L->mpf, L->mask, L->G, A);
+                         L->mpf, L->G, A);
     LAUNCHCHECK();
     c ^= 1;
   }
@@ -2713,11 +2712,11 @@ static void launch_mp_t(slbd_lattice *L, slbd_mp *M, const MPArgs &A) {
   if (!MOVING && L->idx32)
     hipLaunchKernelGGL((k_mpstep<T, NMOM, MOVING, int>), plane_grid(L), dim3(256), 0, L->stream,
                        (const T *)L->pops[L->cur], (const T *)M->q[c], (T *)M->q[c ^ 1], L->mpf,
-                       L->mask, L->objidx, L->tab, L->G, A);
+                       L->objidx, L->tab, L->G, A);
   else
     hipLaunchKernelGGL((k_mpstep<T, NMOM, MOVING, long>), plane_grid(L), dim3(256), 0,
                        L->stream, (const T *)L->pops[L->cur], (const T *)M->q[c],
-                       (T *)M->q[c ^ 1], L->mpf, L->mask, L->objidx, L->tab, L->G, A);
+                       (T *)M->q[c ^ 1], L->mpf, L->objidx, L->tab, L->G, A);
   LAUNCHCHECK();
   M->cur ^= 1;
 }

@@ -5,6 +5,8 @@ Populations after runs against the same number of lbstep calls, bit for bit
 at the edges of its tiles: k tiles with a remainder and rows of one node,
 j and i remainders, planes that are and are not whole population tiles,
 lattices of one plane, odd step counts."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -59,3 +61,43 @@ def test_run_is_single_steps(prec, dims, moving, stokes, skip, bf):
     assert got.s.step == 9
     ref.free()
     got.free()
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("dims,nmom,axis,pads,moving", [
+    ((9, 32, 64), 3, 0, 0.01, 0),
+    ((7, 13, 131), 3, 1, 0.3, 0),     # remainders in j and k, more than one k tile
+    ((70, 6, 11), 3, 2, 0.0, 1),      # many planes; factors with wall terms
+    ((5, 40, 33), 1, 0, 0.2, 0),
+    ((1, 2, 3), 3, 0, 0.01, 0), ((3, 2, 1), 1, 0, 0.0, 0), ((2, 300, 2), 3, 0, 0.01, 0),
+])
+def test_tracer_pairs_are_single_steps(prec, dims, nmom, axis, pads, moving, monkeypatch):
+    """Two tracer steps per pass over the link factors (k_mpstep2, forced)
+    against one (k_mpstep_w): P and the moment sums after 32 and 37 steps, bit
+    for bit; adsorbing sites among the boundary nodes."""
+    out = []
+    print(f"tracer pairs: {dims} prec {prec}", flush=True)
+    for on in "01":
+        monkeypatch.setenv("SLB_MP_STEP2", on)
+        lat = build(dims, prec, moving, 0, 0, 1)
+        L, h = lat.L, lat.h
+        mp = L.newmp(h, b"null")
+        mp.contents.alpha, mp.contents.objects_moving = 0.1, moving
+        L.mpinit(mp)
+        L.mpall(mp, 1.0)
+        L.adsph(mp, 2.5, dims[0] / 2, dims[1] / 2, dims[2] / 2)
+        L.slb_mp_set_adsorption(mp, pads)
+        if nmom > 1:
+            L.slb_mp_track_moments(mp, axis)
+        got = []
+        for n in (32, 37):
+            import sunlightlb_amd as s
+            L.slb_mp_run(mp, n)
+            sums = (C.c_double * 6)()
+            L.slb_mp_sums(mp, sums)
+            L.slb_mp_sync_host(mp)
+            got += [s.view(mp.contents.p, lat.N).copy(), np.array(sums[:])]
+        out.append(got)
+        lat.free()
+    for a, b in zip(*out):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
