@@ -160,8 +160,9 @@ double slb_mp_time_steps(MPSys mp, int nsteps);
 /* ---- batched independent boxes (resistance problems) ---- */
 
 /* A batch of independent periodic boxes, each with nrhs right-hand sides
- * (object velocity sets), stepped together: one kernel launch per step over
- * all problems, the step loop replayed from a captured HIP graph. */
+ * (object velocity sets), stepped together: one kernel launch over all
+ * problems per two steps (SLB_BATCH_STEP2=0: per step), the step loop replayed
+ * from a captured HIP graph. */
 typedef struct slb_batch_s *SLBBatch;
 
 /* New empty batch; prec 32 or 64 (populations; force sums are FP64). */

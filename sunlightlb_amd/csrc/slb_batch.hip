@@ -22,12 +22,15 @@
 #include <string.h>
 #include "slb_dev.h"
 #include "slb_kern.h"
+#include "slb_step2.h"
 
 struct BProb {
   int esi, esj, esk, plane;
   long N;
   long pop_off;   /* first population of this problem in the arena (tiled
                      layout pidx, whole tiles per problem) */
+  int jt, kt, ci; /* two-step tiles of the box (k_bstep2) */
+  long wall_off;  /* first row of the wall terms, -1: walls at rest */
   long node_off;  /* first node of this problem's box in the node tables */
   int tab_off;    /* first object row (9 doubles each) */
   int nobj;
@@ -44,6 +47,19 @@ struct BProb {
  * object's rigid motion) and omega, so that the wall velocity at solid node s
  * is U = w0 + omega x s and only c.U = c.w0 + c.(omega x s) enters a link. */
 #define WROW 8
+
+/* w_l c_l.U of link l with its solid end at (si, sj, sk) on the object of wall
+ * row wr; multiply-adds written out, so that every caller gets the same value */
+template <int l, typename T>
+__device__ __forceinline__ T wall_term(const T *__restrict__ wr, int si, int sj, int sk) {
+#pragma clang fp contract(off)
+  const T sx = T(si), sy = T(sj), sz = T(sk);
+  T cv = T(0);
+  if (CX(l)) cv += T(CX(l)) * __builtin_elementwise_fma(-wr[5], sy, __builtin_elementwise_fma(wr[4], sz, wr[0]));
+  if (CY(l)) cv += T(CY(l)) * __builtin_elementwise_fma(-wr[3], sz, __builtin_elementwise_fma(wr[5], sx, wr[1]));
+  if (CZ(l)) cv += T(CZ(l)) * __builtin_elementwise_fma(-wr[4], sx, __builtin_elementwise_fma(wr[3], sy, wr[2]));
+  return T(WL(l)) * cv;
+}
 
 template <typename T, bool FORCE, int NPT>
 __global__ void __launch_bounds__(512)
@@ -126,13 +142,7 @@ k_bstep(const T *__restrict__ src, T *__restrict__ dst,
                 sj = j - CY(l); sj += (sj < 0) ? P.esj : 0; sj -= (sj >= P.esj) ? P.esj : 0;
                 sk = k - CZ(l); sk += (sk < 0) ? P.esk : 0; sk -= (sk >= P.esk) ? P.esk : 0;
               }
-              const T *wr = wtab + ((long)P.tab_off + oid[sn]) * WROW;
-              const T sx = T(si), sy = T(sj), sz = T(sk);
-              T cv = T(0);
-              if (CX(l)) cv += T(CX(l)) * (wr[0] + wr[4] * sz - wr[5] * sy);
-              if (CY(l)) cv += T(CY(l)) * (wr[1] + wr[5] * sx - wr[3] * sz);
-              if (CZ(l)) cv += T(CZ(l)) * (wr[2] + wr[3] * sy - wr[4] * sx);
-              cu = T(WL(l)) * cv;
+              cu = wall_term<l, T>(wtab + ((long)P.tab_off + oid[sn]) * WROW, si, sj, sk);
             }
             if (FORCE && solid) {
               const double a = (double)v[l];
@@ -170,6 +180,259 @@ k_bstep(const T *__restrict__ src, T *__restrict__ dst,
         if (sacc[q] != 0.0) atomicAdd(acc + 6 * (long)P.acc_off + q, sacc[q]);
       __syncthreads();
     }
+  }
+}
+
+/* ---------------------------------------------------------------------- */
+/* Wall terms.  The wall velocity term of a bounced link, w_l c_l.U, is the  */
+/* same at every step: each node with bounced links of a box gets a place    */
+/* (k_bwall_place), and each moving problem a row of 16 values per place     */
+/* (value l - 1: link l's term, 0 where it does not bounce), so that a step   */
+/* adds one row instead of looking up the solid end's object for each link.  */
+
+__global__ void __launch_bounds__(256)
+k_bwall_place(const uint16_t *__restrict__ flags, long N, int *__restrict__ place,
+              int *__restrict__ count) {
+  const long x = (long)blockIdx.x * 256 + threadIdx.x;
+  const bool has = x < N && (flags[x] & FLAG_LINKS) != 0;
+  const unsigned long long m = __ballot(has);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (lane == 0 && m) base = atomicAdd(count, __popcll(m));
+  base = __shfl(base, 0, 64);
+  if (x < N) place[x] = has ? base + __popcll(m & ((1ULL << lane) - 1)) : -1;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_bwall_fill(const uint16_t *__restrict__ flags, const int32_t *__restrict__ objidx,
+             const int *__restrict__ place, const T *__restrict__ wtab, BProb P,
+             T *__restrict__ rows) {
+  const long xl = (long)blockIdx.x * 256 + threadIdx.x;
+  if (xl >= P.N) return;
+  const int x = (int)xl;
+  const unsigned f = flags[x];
+  if (!(f & FLAG_LINKS)) return;
+  const bool solid = (f & FLAG_SOLID) != 0;
+  const int i = x / P.plane, rem = x - i * P.plane, j = rem / P.esk, k = rem - j * P.esk;
+  const AxisOff32 oi = axis_off32(i, P.esi, P.plane);
+  const AxisOff32 oj = axis_off32(j, P.esj, P.esk);
+  const AxisOff32 ok = axis_off32(k, P.esk, 1);
+  T *row = rows + (P.wall_off + place[x]) * 16;
+  row[14] = row[15] = T(0);
+  Links<1, 15>::run([&](auto LL) {
+    constexpr int l = decltype(LL)::value;
+    T cu = T(0);
+    if ((f >> (l - 1)) & 1u) {
+      int sn = x, si = i, sj = j, sk = k;
+      if (!solid) {
+        sn = x + nb_off<l, -1>(oi, oj, ok);
+        si = i - CX(l); si += (si < 0) ? P.esi : 0; si -= (si >= P.esi) ? P.esi : 0;
+        sj = j - CY(l); sj += (sj < 0) ? P.esj : 0; sj -= (sj >= P.esj) ? P.esj : 0;
+        sk = k - CZ(l); sk += (sk < 0) ? P.esk : 0; sk -= (sk >= P.esk) ? P.esk : 0;
+      }
+      cu = wall_term<l, T>(wtab + ((long)P.tab_off + objidx[sn]) * WROW, si, sj, sk);
+    }
+    row[l - 1] = cu;
+  });
+}
+
+/* Two steps per pass: k_step2 (slb_step2.hip) on the tiles of all problems,
+ * a tile table of (problem, j0, k0, i0), one block each.  What differs: the
+ * collision's parameters are the problem's, and moving walls add their rows.  A row is
+ * loaded with the populations of its plane, and again for the second step,
+ * ahead of the next plane's loads.  Looked up link by link, as k_bstep does,
+ * the terms would be a chain of loads that every wave of the block waits for.
+ * Measured, k_bstep / this kernel: 512 boxes of U{32..64} x 6 right-hand sides
+ * FP32 8.35/5.63 ms per step, FP64 15.25/10.3-11.6; 32 boxes 434/331 us, 6 boxes
+ * of U{28..40} 39/25.5.  NT (non-temporal stores): rows of boxes start off the
+ * 128-byte lines, which tiles share: FP32 without on 6 boxes 25.5 against 35.5
+ * us, on 60 696 against 713; FP64 on 32 boxes 629 against 617 with. */
+/* most threads of a block (FP32 123 registers, FP64 212; FP32 with at most 512:
+ * 392, 768: 344, 1024: 331 us per step on 32 boxes x 6) */
+template <typename T> struct B2Cfg { enum { NTHR = sizeof(T) == 4 ? 1024 : 512 }; };
+
+template <typename T, bool NT>
+__global__ void __launch_bounds__(B2Cfg<T>::NTHR)
+k_bstep2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restrict__ flags,
+         const int *__restrict__ place, const T *__restrict__ rows,
+         const BProb *__restrict__ probs, const int4 *__restrict__ tiles) {
+  typedef T V4 __attribute__((ext_vector_type(4)));
+  constexpr int M1 = B2Cfg<T>::NTHR + 1;
+  __shared__ T buf[2][12 * M1];
+  const int4 td = tiles[blockIdx.x];
+  const BProb P = probs[td.x];
+  const int j0 = td.y, k0 = td.z, i0 = td.w;
+  const int kn = min(P.kt, P.esk - k0), jn = min(P.jt, P.esj - j0), np = min(P.ci, P.esi - i0);
+  const int S = P.kt + 2, main = (P.jt + 2) * P.kt;
+  const int q = (int)threadIdx.x;
+  const int row = q < main ? q / P.kt : (q - main) >> 1;
+  const int col = q < main ? 1 + q - row * P.kt : ((q - main) & 1) ? kn + 1 : 0;
+  const bool valid = row <= jn + 1 && col <= kn + 1;
+  const bool out = valid && row >= 1 && row <= jn && col >= 1 && col <= kn;
+  if (!__any(valid)) {     /* a wave past the tile only keeps the barriers */
+    for (int st = 0; st < np + 2; st++) lds_barrier();
+    return;
+  }
+  const int lidx = valid ? row * S + col : M1 - 1;
+  const int j = (j0 + min(row, jn + 1) - 1 + P.esj) % P.esj;
+  const int k = (k0 + min(col, kn + 1) - 1 + P.esk) % P.esk;
+  const int t0 = j * P.esk + k;
+  const T *s = src + P.pop_off;
+  T *d = dst + P.pop_off;
+  const uint16_t *fl = flags + P.node_off;
+  const int *pl_of = place + P.node_off;
+  const T *wr = rows + P.wall_off * 16;
+  const bool moving = P.wall_off >= 0;
+  PhysArgs A;
+  A.omega = P.omega; A.comega = P.comega; A.rho0 = P.rho0;
+  A.stokes = P.stokes; A.skip_solid = P.skip_solid;
+  A.bfx = P.bf[0]; A.bfy = P.bf[1]; A.bfz = P.bf[2];
+  uint32_t off[9];         /* in-plane byte of (j - cy, k - cz): index 3 (cy + 1) + cz + 1 */
+  {
+    const AxisOff32 oj = axis_off32(j, P.esj, P.esk), ok = axis_off32(k, P.esk, 1);
+#pragma unroll
+    for (int c = 0; c < 9; c++)
+      off[c] = (uint32_t)(t0 + (c / 3 == 0 ? oj.p : c / 3 == 2 ? oj.m : 0) +
+                          (c % 3 == 0 ? ok.p : c % 3 == 2 ? ok.m : 0)) * (uint32_t)sizeof(T);
+  }
+  auto uni = [](int i) { return __builtin_amdgcn_readfirstlane(i); };
+  auto wrap = [&](int i) { return i < 0 ? i + P.esi : (i >= P.esi ? i - P.esi : i); };
+  auto bit = [](unsigned f, int l) { return (int)(f << (32 - l)) >> 31; };
+  auto pick = [&](unsigned f, int l, T x, T y) -> T {
+    const int m = bit(f, l);
+    if constexpr (sizeof(T) == 4) {
+      return __int_as_float((__float_as_int(x) & m) | (__float_as_int(y) & ~m));
+    } else {
+      return __hiloint2double((__double2hiint(x) & m) | (__double2hiint(y) & ~m),
+                              (__double2loint(x) & m) | (__double2loint(y) & ~m));
+    }
+  };
+  /* byte offset of population 0 of the node at byte n of a plane array */
+  auto tiled = [&](int pl, uint32_t o) -> uint32_t {
+    return pop_byte<T>((uint32_t)(pl * P.plane) * (uint32_t)sizeof(T) + o);
+  };
+  auto load = [&](T (&v)[15], int pm, int pl, int pp, unsigned f) {
+    const uint32_t o0 = tiled(pl, off[4]);
+    Links<0, 15>::run([&](auto LL) {
+      constexpr int l = decltype(LL)::value;
+      constexpr int c = 3 * (CY(l) + 1) + CZ(l) + 1;
+      const int bb = l > 0 ? bit(f, l) : 0;
+      /* both offsets from the lower of the two populations' runs: never negative */
+      constexpr int lo = l < OPP(l) ? l : OPP(l);
+      const uint32_t pulled = (l ? tiled(CX(l) > 0 ? pm : CX(l) < 0 ? pp : pl, off[c]) : o0) +
+                              (uint32_t)((l - lo) * POP_TILE * (long)sizeof(T));
+      const uint32_t own = o0 + (uint32_t)((OPP(l) - lo) * POP_TILE * (long)sizeof(T));
+      v[l] = *(const T *)((const char *)(s + lo * POP_TILE) + ((own & bb) | (pulled & ~bb)));
+    });
+  };
+  auto node = [&](int pl) { return pl * P.plane + t0; };
+  auto walls = [&](T (&r)[16], unsigned f, int at) {
+    if (f & FLAG_LINKS) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const V4 v = *(const V4 *)(wr + (long)at * 16 + 4 * c);
+        r[4 * c] = v[0]; r[4 * c + 1] = v[1]; r[4 * c + 2] = v[2]; r[4 * c + 3] = v[3];
+      }
+    }
+  };
+  auto update = [&](T (&v)[15], const T (&r)[16], unsigned f) {
+    const bool solid = (f & FLAG_SOLID) != 0;
+    if (moving && (f & FLAG_LINKS)) {
+#pragma unroll
+      for (int l = 1; l < 15; l++) v[l] += r[l - 1];
+    }
+    if (!(A.skip_solid && solid)) {
+      T jbx = T(0), jby = T(0), jbz = T(0);
+      if (!solid) { jbx = T(A.bfx); jby = T(A.bfy); jbz = T(A.bfz); }
+      collide_node<T>(v, jbx, jby, jbz, A);
+    }
+  };
+  T va[15], vb[15], a[15], dg[4], o[5];
+  T ra[16], rb[16];        /* wall rows of plane pl, and of plane pl - 1 again */
+  int pm = uni(wrap(i0 - 2 + P.esi)), pl = uni(wrap(i0 - 1)), pp = uni(i0);
+  unsigned f = fl[node(pl)], fn = fl[node(pp)], fp = 0;
+  int w = 0, wn = 0, wp = 0;   /* places in the wall rows */
+  if (moving) {
+    w = (f & FLAG_LINKS) ? pl_of[node(pl)] : 0;
+    wn = (fn & FLAG_LINKS) ? pl_of[node(pp)] : 0;
+  }
+#pragma unroll
+  for (int c = 0; c < 16; c++) { ra[c] = T(0); rb[c] = T(0); }
+  load(va, pm, pl, pp, f);
+  if (moving) walls(ra, f, w);
+#pragma unroll
+  for (int l = 0; l < 15; l++) a[l] = T(0);
+#pragma unroll
+  for (int m = 0; m < 4; m++) dg[m] = T(0);
+#pragma unroll
+  for (int m = 0; m < 5; m++) o[m] = T(0);
+  int p2 = uni(wrap(pp + 1));
+  unsigned f2 = fl[node(p2)];  /* flags run one plane further ahead than the populations */
+  auto plane = [&](T (&v)[15], T (&nv)[15], T *B, int st) {
+    const int p3 = uni(wrap(p2 + 1));
+    unsigned f3 = 0;
+    int w2 = 0;
+    update(v, ra, f);
+    Links<3, 15>::run([&](auto LL) {
+      constexpr int l = decltype(LL)::value;
+      B[XSLOT(l) * M1 + lidx] = v[l];
+    });
+    if (moving && st >= 2) walls(rb, fp, wp);
+    if (st < np + 1) {
+      load(nv, pl, pp, p2, fn);
+      f3 = fl[node(p3)];
+      if (moving) {
+        walls(ra, fn, wn);
+        if (f2 & FLAG_LINKS) w2 = pl_of[node(p2)];
+      }
+    }
+    lds_barrier();
+    if (out) {
+      auto pull = [&](auto LL) -> T {
+        constexpr int l = decltype(LL)::value;
+        return B[XSLOT(l) * M1 + lidx - CY(l) * S - CZ(l)];
+      };
+      if (st >= 2) {
+        a[2] = pick(fp, 2, o[0], v[2]);
+        a[8] = pick(fp, 8, o[4], pull(std::integral_constant<int, 8>{}));
+        a[10] = pick(fp, 10, o[3], pull(std::integral_constant<int, 10>{}));
+        a[12] = pick(fp, 12, o[2], pull(std::integral_constant<int, 12>{}));
+        a[14] = pick(fp, 14, o[1], pull(std::integral_constant<int, 14>{}));
+        update(a, rb, fp);
+        const uint32_t o0 = tiled(pm, off[4]);
+        Links<0, 15>::run([&](auto LL) {
+          constexpr int l = decltype(LL)::value;
+          T *p = (T *)((char *)(d + l * POP_TILE) + o0);
+          if constexpr (NT) __builtin_nontemporal_store(a[l], p);
+          else *p = a[l];
+        });
+      }
+      a[0] = v[0];
+      a[1] = pick(f, 1, v[2], o[0]);
+      a[7] = pick(f, 7, v[14], dg[0]);
+      a[9] = pick(f, 9, v[12], dg[1]);
+      a[11] = pick(f, 11, v[10], dg[2]);
+      a[13] = pick(f, 13, v[8], dg[3]);
+      a[3] = pick(f, 3, v[4], pull(std::integral_constant<int, 3>{}));
+      a[4] = pick(f, 4, v[3], pull(std::integral_constant<int, 4>{}));
+      a[5] = pick(f, 5, v[6], pull(std::integral_constant<int, 5>{}));
+      a[6] = pick(f, 6, v[5], pull(std::integral_constant<int, 6>{}));
+      dg[0] = pull(std::integral_constant<int, 7>{});
+      dg[1] = pull(std::integral_constant<int, 9>{});
+      dg[2] = pull(std::integral_constant<int, 11>{});
+      dg[3] = pull(std::integral_constant<int, 13>{});
+      o[0] = v[1]; o[1] = v[7]; o[2] = v[9]; o[3] = v[11]; o[4] = v[13];
+    }
+    fp = f; f = fn; fn = f2; f2 = f3;
+    wp = w; w = wn; wn = w2;
+    pm = pl; pl = pp; pp = p2; p2 = p3;
+  };
+  for (int st = 0;;) {
+    plane(va, vb, buf[0], st);
+    if (++st == np + 2) break;
+    plane(vb, va, buf[1], st);
+    if (++st == np + 2) break;
   }
 }
 
@@ -226,6 +489,12 @@ struct slbd_batch {
   int2 *tiles;
   int nprob, ntiles, nacc;
   long nnodes_total, npop_total, nnode_tab;
+  /* two steps per pass: places and rows of the wall terms, tile table */
+  int pairs;
+  int *place;
+  void *wrows;
+  int4 *tiles2;
+  int ntiles2, thr2;        /* tiles, threads per block */
   BProb *hprobs;
   int *box_first_prob;
   /* launch configuration */
@@ -317,6 +586,97 @@ static void build_tiles(slbd_batch *B) {
   invalidate_graphs(B);
 }
 
+/* Two steps per pass: tiles of every box (the split of a plane that costs
+ * least, as slbd_step2_plan) in chunks along i, and the wall terms. */
+static void plan_pairs(slbd_batch *B) {
+  const char *e = getenv("SLB_BATCH_STEP2");
+  B->pairs = !(e && atoi(e) == 0);
+  for (int p = 0; p < B->nprob; p++)   /* 32-bit byte offsets in a problem */
+    if (15 * pop_nodes(B->hprobs[p].N) * (long)bts(B->prec) >= (1L << 32)) B->pairs = 0;
+  if (!B->pairs) return;
+  const int cap = B->prec == 32 ? B2Cfg<float>::NTHR : B2Cfg<double>::NTHR;
+  const int cus = 256;
+  int pts = 0;
+  long best = 0, total[4] = {0, 0, 0, 0}, longest[4] = {0, 0, 0, 0};
+  for (int p = 0; p < B->nprob; p++) {
+    BProb *q = &B->hprobs[p];
+    double bc = 0.0;
+    q->jt = 0;
+    for (int nk = 1; nk <= (q->esk + 31) / 32 || q->jt == 0; nk++) {
+      const int kt = (q->esk + nk - 1) / nk, nkt = (q->esk + kt - 1) / kt;
+      for (int jq = 1; jq <= q->esj && (jq + 2) * (kt + 2) <= cap; jq++) {
+        const int njt = (q->esj + jq - 1) / jq, jt = (q->esj + njt - 1) / njt;
+        const double cost = (1.0 + 16.0 / kt) * njt * nkt *
+                            ((double)(jt + 2) * (kt + 2) + (double)jt * kt + 1000.0);
+        if (q->jt == 0 || cost < bc) { bc = cost; q->jt = jt; q->kt = kt; }
+      }
+    }
+    if ((q->jt + 2) * (q->kt + 2) > pts) pts = (q->jt + 2) * (q->kt + 2);
+    const long t = (long)((q->esj + q->jt - 1) / q->jt) * ((q->esk + q->kt - 1) / q->kt);
+    for (int c = 0; c < 4; c++) {
+      const int ci = (q->esi + c) / (c + 1);
+      total[c] += t * ((q->esi + ci - 1) / ci);
+      if (ci + 2 > longest[c]) longest[c] = ci + 2;
+    }
+  }
+  for (int c = 1; c < 4; c++)
+    if ((total[c] + cus - 1) / cus * longest[c] < (total[best] + cus - 1) / cus * longest[best])
+      best = c;
+  int4 *h = (int4 *)malloc(sizeof(int4) * (total[best] > 0 ? total[best] : 1));
+  long n = 0;
+  for (int p = 0; p < B->nprob; p++) {
+    BProb *q = &B->hprobs[p];
+    q->ci = (int)((q->esi + best) / (best + 1));
+    for (int i0 = 0; i0 < q->esi; i0 += q->ci)
+      for (int j0 = 0; j0 < q->esj; j0 += q->jt)
+        for (int k0 = 0; k0 < q->esk; k0 += q->kt) h[n++] = make_int4(p, j0, k0, i0);
+  }
+  B->ntiles2 = (int)n;
+  B->thr2 = (pts + 63) & ~63;
+  HIPCHECK(hipMalloc(&B->tiles2, sizeof(int4) * (n > 0 ? n : 1)));
+  HIPCHECK(hipMemcpy(B->tiles2, h, sizeof(int4) * n, hipMemcpyHostToDevice));
+  free(h);
+  /* places of the boxes' boundary nodes, then the moving problems' rows */
+  int *cnt, *hc = (int *)calloc(B->nbox, sizeof(int));
+  HIPCHECK(hipMalloc(&B->place, sizeof(int) * B->nnode_tab));
+  HIPCHECK(hipMalloc(&cnt, sizeof(int) * B->nbox));
+  HIPCHECK(hipMemsetAsync(cnt, 0, sizeof(int) * B->nbox, B->stream));
+  long nrow = 0;
+  for (int b = 0; b < B->nbox; b++) {
+    const BProb *q = &B->hprobs[B->box_first_prob[b]];
+    if (!B->box[b].moving) continue;
+    hipLaunchKernelGGL(k_bwall_place, dim3((unsigned)((q->N + 255) / 256)), dim3(256), 0, B->stream,
+                       B->flags + q->node_off, q->N, B->place + q->node_off, cnt + b);
+    LAUNCHCHECK();
+  }
+  HIPCHECK(hipMemcpyAsync(hc, cnt, sizeof(int) * B->nbox, hipMemcpyDeviceToHost, B->stream));
+  HIPCHECK(hipStreamSynchronize(B->stream));
+  HIPCHECK(hipFree(cnt));
+  for (int b = 0; b < B->nbox; b++)
+    if (B->box[b].moving)
+      for (int r = 0; r < B->box[b].nrhs; r++) {
+        B->hprobs[B->box_first_prob[b] + r].wall_off = nrow;
+        nrow += hc[b];
+      }
+  free(hc);
+  HIPCHECK(hipMalloc(&B->wrows, bts(B->prec) * 16 * (nrow > 0 ? nrow : 1)));
+  for (int p = 0; p < B->nprob; p++) {
+    const BProb *q = &B->hprobs[p];
+    if (q->wall_off < 0) continue;
+    const dim3 g((unsigned)((q->N + 255) / 256));
+    if (B->prec == 32)
+      hipLaunchKernelGGL(k_bwall_fill<float>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
+                         B->objidx + q->node_off, B->place + q->node_off, (const float *)B->wtab, *q,
+                         (float *)B->wrows);
+    else
+      hipLaunchKernelGGL(k_bwall_fill<double>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
+                         B->objidx + q->node_off, B->place + q->node_off, (const double *)B->wtab,
+                         *q, (double *)B->wrows);
+    LAUNCHCHECK();
+  }
+  HIPCHECK(hipStreamSynchronize(B->stream));
+}
+
 extern "C" int slbd_batch_commit(slbd_batch *B) {
   if (B->committed || B->nbox == 0) return -1;
   int nprob = 0, nacc = 0;
@@ -385,6 +745,7 @@ extern "C" int slbd_batch_commit(slbd_batch *B) {
       q->moving = x->moving; q->stokes = x->stokes; q->skip_solid = x->skip_solid;
       q->omega = 1.0 / x->tau; q->comega = 1.0 - q->omega; q->rho0 = x->rho0;
       for (int c = 0; c < 3; c++) q->bf[c] = x->bf[c];
+      q->wall_off = -1;
       pop_off += 15 * pop_nodes(N);
     }
     node_off += N;
@@ -405,6 +766,7 @@ extern "C" int slbd_batch_commit(slbd_batch *B) {
   free(hw);
   HIPCHECK(hipStreamSynchronize(B->stream));
   HIPCHECK(hipFree(dmask));
+  plan_pairs(B);
   HIPCHECK(hipMalloc(&B->probs, sizeof(BProb) * nprob));
   HIPCHECK(hipMemcpy(B->probs, B->hprobs, sizeof(BProb) * nprob, hipMemcpyHostToDevice));
   long tot = 0;
@@ -446,6 +808,29 @@ static void bstep(slbd_batch *B, bool force) {
   if (B->prec == 32) blaunch<float>(B, force); else blaunch<double>(B, force);
 }
 
+template <typename T, bool NT>
+static void bstep2_t(slbd_batch *B) {
+  hipLaunchKernelGGL((k_bstep2<T, NT>), dim3((unsigned)B->ntiles2), dim3((unsigned)B->thr2), 0,
+                     B->stream, (const T *)B->pops[B->cur], (T *)B->pops[B->cur ^ 1], B->flags,
+                     B->place, (const T *)B->wrows, B->probs, B->tiles2);
+  LAUNCHCHECK();
+  B->cur ^= 1;
+}
+
+static void bstep2(slbd_batch *B) {
+  if (B->prec == 32) bstep2_t<float, false>(B);
+  else if (16 * B->npop_total > 256000000L) bstep2_t<double, true>(B);
+  else bstep2_t<double, false>(B);
+}
+
+/* nsteps plain steps; pairs: two per launch as far as they go */
+static void bsteps(slbd_batch *B, int nsteps, bool pairs) {
+  int s = 0;
+  if (pairs)
+    for (; s + 2 <= nsteps; s += 2) bstep2(B);
+  for (; s < nsteps; s++) bstep(B, false);
+}
+
 extern "C" void slbd_batch_config(slbd_batch *B, int block, int npt, int grid) {
   if (block != 64 && block != 128 && block != 256 && block != 512) block = 256;
   if (npt != 1 && npt != 2 && npt != 4) npt = 1;
@@ -455,14 +840,15 @@ extern "C" void slbd_batch_config(slbd_batch *B, int block, int npt, int grid) {
 
 #define BATCH_GRAPH_STEPS 32
 
-/* Capture BATCH_GRAPH_STEPS steps starting from the live buffer B->cur. */
+/* Capture BATCH_GRAPH_STEPS steps (a multiple of 4: as single steps or in pairs
+ * they end on the buffer they began on) starting from the live buffer B->cur. */
 static void build_graph(slbd_batch *B) {
   if (B->tiled_block != B->block || B->tiled_npt != B->npt) build_tiles(B);
   const int cur0 = B->cur;
   if (B->graph_valid[cur0]) return;
   hipGraph_t g;
   HIPCHECK(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-  for (int s = 0; s < BATCH_GRAPH_STEPS; s++) bstep(B, false);
+  bsteps(B, BATCH_GRAPH_STEPS, B->pairs != 0);
   HIPCHECK(hipStreamEndCapture(B->stream, &g));
   HIPCHECK(hipGraphInstantiate(&B->gexec[cur0], g, NULL, NULL, 0));
   HIPCHECK(hipGraphDestroy(g));
@@ -481,7 +867,8 @@ extern "C" void slbd_batch_run(slbd_batch *B, int nsteps, int use_graph) {
     for (; s + BATCH_GRAPH_STEPS <= nsteps; s += BATCH_GRAPH_STEPS)
       HIPCHECK(hipGraphLaunch(B->gexec[B->cur], B->stream));
   }
-  for (; s < nsteps; s++) bstep(B, false);
+  /* use_graph 0: the autotuner times the single-step launch shapes */
+  bsteps(B, nsteps - s, B->pairs != 0 && use_graph != 0);
 }
 
 extern "C" double slbd_batch_time(slbd_batch *B, int nsteps, int use_graph) {
@@ -568,7 +955,7 @@ extern "C" void slbd_batch_destroy(slbd_batch *B) {
   HIPCHECK(hipStreamSynchronize(B->stream));
   invalidate_graphs(B);
   void *ps[] = {B->pops[0], B->pops[1], B->flags, B->objidx, B->tab, B->wtab, B->acc, B->probs,
-                B->tiles};
+                B->tiles, B->place, B->wrows, B->tiles2};
   for (size_t q = 0; q < sizeof ps / sizeof ps[0]; q++)
     if (ps[q]) HIPCHECK(hipFree(ps[q]));
   for (int b = 0; b < B->nbox; b++) { free(B->box[b].objidx); free(B->box[b].mask); free(B->box[b].tab); }

@@ -1443,9 +1443,11 @@ extern "C" const char *slbd_arch(void) {
  * or the environment names a single-step kernel or 64-bit indices.  Lattices
  * beyond 32-bit population indices need planes of whole population tiles.
  * Stores are non-temporal except where both buffers fit the 256 MB last-level
- * cache and exceed the L2s by far, and the next pass reads them there: nt /
+ * cache and exceed the L2s by far, and the next pass reads them there, and
+ * where rows start off a 128-byte line, and two tiles share its lines: nt /
  * plain us per FP32 step at 96^3 (106 MB) 15.8/12.6, 128^3 (252 MB)
- * 31.9/30.4, 160^3 (491 MB) 58.8/61.5, 64^3 (31 MB) 6.05/6.31. */
+ * 31.9/30.4, 160^3 (491 MB) 58.8/61.5, 64^3 (31 MB) 6.05/6.31; off the line
+ * 200^3 152/141, 400^3 1519/1258. */
 static void pair_policy(slbd_lattice *L) {
   const long np = 15 * pop_nodes(L->N), ts = (long)tsize(L->prec);
   const char *e = getenv("SLB_STEP2");
@@ -1454,7 +1456,9 @@ static void pair_policy(slbd_lattice *L) {
              (small || (L->G.plane % POP_TILE == 0 && 15L * L->G.plane * ts < (1L << 32))) &&
              slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2);
   const double both = 30.0 * (double)L->N * (double)ts;
-  L->pair_nt = L->G.nt_store && !(both > 64e6 && both <= 256e6);
+  const bool lines = ((long)L->esk * ts) % 128 == 0 &&
+                     (L->plan2.nkt == 1 || ((long)L->plan2.kt * ts) % 128 == 0);
+  L->pair_nt = L->G.nt_store && lines && !(both > 64e6 && both <= 256e6);
 }
 
 /* The step kernel of a lattice, from its shape and precision (made again

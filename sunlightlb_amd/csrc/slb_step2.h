@@ -1,11 +1,36 @@
 /*
- * slb_step2.h -- interface of the two-step kernel (slb_step2.hip) to the
- * single-lattice path (slb_dev.hip).
+ * slb_step2.h -- the two-step kernel (slb_step2.hip): what the batched one
+ * (slb_batch.hip) shares, and its interface to the single-lattice path
+ * (slb_dev.hip).
  */
 #ifndef SLB_STEP2_H
 #define SLB_STEP2_H
 
 #include "slb_kern.h"
+
+/* LDS slot of a population that leaves its column: c_x = -1 diagonals, c_x =
+ * 0 axes, c_x = +1 diagonals */
+__host__ __device__ constexpr int XSLOT(int l) {
+  return l == 8 ? 0 : l == 10 ? 1 : l == 12 ? 2 : l == 14 ? 3
+       : l == 3 ? 4 : l == 4 ? 5 : l == 5 ? 6 : l == 6 ? 7
+       : l == 7 ? 8 : l == 9 ? 9 : l == 11 ? 10 : 11;
+}
+
+/* byte offset of a node's population 0 in the tiled layout, from the byte
+ * offset n of the node in an array of one T per node: a shift and a
+ * multiply-add (population l: l tiles further) */
+template <typename T>
+__device__ __forceinline__ uint32_t pop_byte(uint32_t n) {
+  constexpr int SH = POP_SHIFT + (sizeof(T) == 4 ? 2 : 3);
+  return n + (n >> SH) * (uint32_t)(14 * POP_TILE * sizeof(T));
+}
+
+__device__ __forceinline__ void lds_barrier() {
+  /* orders LDS only: the next plane's global loads stay in flight */
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 /* jt x kt nodes of a plane per block, ci planes; their counts */
 struct Step2Plan {

@@ -39,25 +39,11 @@
 #include "slb_kern.h"
 #include "slb_step2.h"
 
-/* LDS slot of a population that leaves its column: c_x = -1 diagonals, c_x =
- * 0 axes, c_x = +1 diagonals */
-__host__ __device__ constexpr int XSLOT(int l) {
-  return l == 8 ? 0 : l == 10 ? 1 : l == 12 ? 2 : l == 14 ? 3
-       : l == 3 ? 4 : l == 4 ? 5 : l == 5 ? 6 : l == 6 ? 7
-       : l == 7 ? 8 : l == 9 ? 9 : l == 11 ? 10 : 11;
-}
-
-__device__ __forceinline__ void lds_barrier() {
-  /* orders LDS only: the next plane's global loads stay in flight */
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 /* MODE 0: planes of whole population tiles (plane % 1024 == 0) and buffers
  * under 4 GB: a column's in-plane byte offset is fixed and a plane adds a
- * scalar; MODE 1: any plane, 32-bit population indices; MODE 2: as 0 with
- * 64-bit plane offsets.  NT: non-temporal stores. */
+ * scalar; MODE 1: any plane, buffers under 4 GB (two more operations per
+ * load); MODE 2: as 0 with 64-bit plane offsets; MODE 3: any plane, 32-bit
+ * population indices.  NT: non-temporal stores. */
 template <typename T, int BF, int MODE, bool NT>
 __global__ void __launch_bounds__(Step2Cfg<T>::NTHR)
 k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restrict__ flags,
@@ -95,7 +81,9 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
     for (int c = 0; c < 9; c++) {
       const int t = t0 + (c / 3 == 0 ? oj.p : c / 3 == 2 ? oj.m : 0) +
                     (c % 3 == 0 ? ok.p : c % 3 == 2 ? ok.m : 0);
-      off[c] = MODE == 1 ? (uint32_t)t : (uint32_t)pidx32(0, t) * (uint32_t)sizeof(T);
+      off[c] = MODE == 3 ? (uint32_t)t
+               : MODE == 1 ? (uint32_t)t * (uint32_t)sizeof(T)
+                           : (uint32_t)pidx32(0, t) * (uint32_t)sizeof(T);
     }
   }
   auto uni = [](int i) { return __builtin_amdgcn_readfirstlane(i); };
@@ -115,6 +103,7 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
   /* the 15 populations that stream into the column's node of plane pl (pm
    * and pp its neighbours): bounced links take the node's own opposite */
   auto load = [&](T (&v)[15], int pm, int pl, int pp, unsigned f) {
+    const uint32_t o0 = MODE == 1 ? pop_byte<T>((uint32_t)pl * (uint32_t)G.plane * (uint32_t)sizeof(T) + off[4]) : 0;
     Links<0, 15>::run([&](auto LL) {
       constexpr int l = decltype(LL)::value;
       constexpr int c = 3 * (CY(l) + 1) + CZ(l) + 1;
@@ -128,6 +117,14 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
             ((uint32_t)pl * pitch + (uint32_t)(OPP(l) * POP_TILE)) * (uint32_t)sizeof(T) + off[4];
         v[l] = *(const T *)((const char *)src + ((own & bb) | (pulled & ~bb)));
       } else if constexpr (MODE == 1) {
+        /* both offsets from the lower of the two populations' runs: never negative */
+        constexpr int lo = l < OPP(l) ? l : OPP(l);
+        const uint32_t pulled =
+            pop_byte<T>((uint32_t)ps * (uint32_t)G.plane * (uint32_t)sizeof(T) + off[c]) +
+            (uint32_t)((l - lo) * POP_TILE * (long)sizeof(T));
+        const uint32_t own = o0 + (uint32_t)((OPP(l) - lo) * POP_TILE * (long)sizeof(T));
+        v[l] = *(const T *)((const char *)(src + lo * POP_TILE) + ((own & bb) | (pulled & ~bb)));
+      } else if constexpr (MODE == 3) {
         const int o = bb ? pidx32(OPP(l), pl * G.plane + (int)off[4])
                          : pidx32(l, ps * G.plane + (int)off[c]);
         v[l] = src[o];
@@ -196,6 +193,7 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
         a[12] = pick(fp, 12, o[2], pull(std::integral_constant<int, 12>{}));
         a[14] = pick(fp, 14, o[1], pull(std::integral_constant<int, 14>{}));
         update(a, pm, fp);
+        const uint32_t o0 = MODE == 1 ? pop_byte<T>((uint32_t)pm * (uint32_t)G.plane * (uint32_t)sizeof(T) + off[4]) : 0;
         Links<0, 15>::run([&](auto LL) {
           constexpr int l = decltype(LL)::value;
           T *p;
@@ -203,6 +201,8 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
             p = (T *)((char *)dst + (((uint32_t)pm * (15u * (uint32_t)G.plane) +
                                       (uint32_t)(l * POP_TILE)) * (uint32_t)sizeof(T) + off[4]));
           else if constexpr (MODE == 1)
+            p = (T *)((char *)(dst + l * POP_TILE) + o0);
+          else if constexpr (MODE == 3)
             p = dst + pidx32(l, pm * G.plane + t0);
           else
             p = (T *)((char *)(dst + ((long)pm * (15L * G.plane) + l * POP_TILE)) + off[4]);
@@ -297,12 +297,15 @@ static void launch2(const Step2Args *a, const PhysArgs &A, const Geom &G, hipStr
 template <typename T>
 static void launch2_t(const Step2Args *a, const PhysArgs &A, const Geom &G, hipStream_t st) {
   const bool whole = G.plane % POP_TILE == 0;
-  if (whole && 15 * pop_nodes(G.N) * (long)sizeof(T) < (1L << 32)) {
+  const bool small = 15 * pop_nodes(G.N) * (long)sizeof(T) < (1L << 32);
+  if (whole && small) {
     if (a->nt) launch2<T, 0, true>(a, A, G, st); else launch2<T, 0, false>(a, A, G, st);
   } else if (whole) {
     launch2<T, 2, true>(a, A, G, st);
-  } else {
+  } else if (small) {
     if (a->nt) launch2<T, 1, true>(a, A, G, st); else launch2<T, 1, false>(a, A, G, st);
+  } else {
+    launch2<T, 3, true>(a, A, G, st);
   }
 }
 

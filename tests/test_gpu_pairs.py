@@ -101,3 +101,54 @@ def test_tracer_pairs_are_single_steps(prec, dims, nmom, axis, pads, moving, mon
         lat.free()
     for a, b in zip(*out):
         assert np.all(np.isfinite(a)) and np.array_equal(a, b)
+
+
+BATCH = [  # dims, objects moving, stokes, skip_solid, body force
+    ((33, 31, 29), 1, 1, 0, 0), ((12, 40, 64), 0, 0, 1, 1), ((5, 3, 701), 1, 0, 0, 1), ((2, 2, 2), 1, 1, 0, 1),
+    ((1, 1, 7), 0, 1, 0, 1), ((70, 4, 5), 1, 0, 1, 0), ((3, 120, 1), 1, 1, 0, 1),
+]
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+def test_batch_pairs_are_single_steps(prec, monkeypatch):
+    """A batch in pairs (k_bstep2, wall terms from their rows) against single
+    steps (k_bstep): populations after 33 and 2 steps, bit for bit, on boxes at
+    the edges of its tiles; forces of measure() to the order of their atomics."""
+    out = []
+    for on in "01":
+        monkeypatch.setenv("SLB_BATCH_STEP2", on)
+        print(f"batch pairs: prec {prec} pairs {on}", flush=True)
+        b, nobj = None, []
+        for q, (dims, moving, stokes, skip, bf) in enumerate(BATCH):
+            lat = build(dims, prec, moving, stokes, skip, bf)
+            if b is None:
+                b = lat.L.slb_batch_new(prec)
+            n = len(lat.objects())
+            vel = np.random.default_rng(q).normal(0, 0.01, (2, n, 6)) if moving else None
+            assert lat.L.slb_batch_add(b, lat.h, 2, vel.ctypes.data_as(C.POINTER(C.c_double))
+                                       if moving else None) == q
+            nobj.append(n)
+            L = lat.L
+            lat.free()
+        assert L.slb_batch_commit(b) == 0
+        got = []
+        for n in (33, 2):
+            L.slb_batch_run(b, n)
+            for q, (dims, *_) in enumerate(BATCH):
+                for r in range(2):
+                    a = np.zeros(15 * int(np.prod(dims)))
+                    L.slb_batch_get_pops(b, q, r, a.ctypes.data_as(C.POINTER(C.c_double)))
+                    got.append(a)
+        L.slb_batch_measure(b)
+        frc = []
+        for q, n in enumerate(nobj):
+            f, t = np.zeros(3 * max(n, 1)), np.zeros(3 * max(n, 1))
+            assert L.slb_batch_forces(b, q, 1, f.ctypes.data_as(C.POINTER(C.c_double)),
+                                      t.ctypes.data_as(C.POINTER(C.c_double))) == n
+            frc.append(np.concatenate([f, t]))
+        out.append((got, frc))
+        L.slb_batch_free(b)
+    for a, c in zip(out[0][0], out[1][0]):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, c)
+    for a, c in zip(out[0][1], out[1][1]):
+        assert np.abs(a - c).max() <= 1e-12 * max(np.abs(a).max(), 1e-30)
