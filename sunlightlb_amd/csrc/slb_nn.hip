@@ -78,11 +78,17 @@ __device__ __forceinline__ int tap_node(const NGeom &G, int z, int y, int x, int
 /* weights are loaded once and applied to all NTW tiles, whose NTW input     */
 /* loads are in flight together.                                            */
 
-template <int MT, int NTW>
+/* CI: the input channels where they are 16, 32 or 64 (taps without divisions,
+ * two K chunks' loads in flight), else 0.  Bound by the latency of a chunk's
+ * loads on few nodes: 64 -> 64 channels on 1080 and 8640 nodes 51 -> 34 us with
+ * CI and one tile per wave, 16 -> 16 on 553 thousand nodes 46 -> 43 us.  The K
+ * order and MFMA sequence per tile do not depend on CI or NTW. */
+template <int MT, int NTW, int CI>
 __global__ void __launch_bounds__(256)
-k_conv(const uint16_t *__restrict__ X, int Cin, const uint16_t *__restrict__ W, int Kp,
+k_conv(const uint16_t *__restrict__ X, int cin, const uint16_t *__restrict__ W, int kpad,
        const float *__restrict__ bias, uint16_t *__restrict__ Y, float *__restrict__ Yf,
        int Cout, int relu, int sgn, NGeom G) {
+  const int Cin = CI ? CI : cin, Kp = CI ? (27 * CI + 31) / 32 * 32 : kpad;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int n0 = (blockIdx.x * 4 + wv) * 16 * NTW;
   if (n0 >= G.N) return;
@@ -103,6 +109,7 @@ k_conv(const uint16_t *__restrict__ X, int Cin, const uint16_t *__restrict__ W, 
   for (int u = 0; u < NTW; u++)
 #pragma unroll
     for (int m = 0; m < MT; m++) acc[u][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll(CI ? 2 : 1)
   for (int k0 = 0; k0 < Kp; k0 += 32) {
     const int kk = k0 + 8 * grp;
     /* the weights of this K chunk, loaded once for all NTW node tiles */
@@ -1100,15 +1107,32 @@ extern "C" void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const f
     LAUNCHCHECK();
     return;
   }
-#define SLBN_CONV(MT)                                                                      \
-  hipLaunchKernelGGL((k_conv<MT, SLBN_CONV_NTW>), dim3(g), dim3(256), 0, nn_stream, X, cin, W, \
-                     Kp, bias, Y, Yf, \
-                     cout, relu, sgn, G)
+  /* few nodes: one tile per wave, for four times the blocks (64 -> 64 channels
+   * on 1080 nodes: 5 blocks of four tiles per wave) */
+  const bool few = g < 512;
+  const unsigned gf = few ? blocks_for(G.N, 64) : g;
+#define SLBN_CONVC(MT, CI)                                                                       \
+  do {                                                                                           \
+    if (few)                                                                                     \
+      hipLaunchKernelGGL((k_conv<MT, 1, CI>), dim3(gf), dim3(256), 0, nn_stream, X, cin, W, Kp,  \
+                         bias, Y, Yf, cout, relu, sgn, G);                                       \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_conv<MT, SLBN_CONV_NTW, CI>), dim3(g), dim3(256), 0, nn_stream, X,   \
+                         cin, W, Kp, bias, Y, Yf, cout, relu, sgn, G);                           \
+  } while (0)
+#define SLBN_CONV(MT)                                                                            \
+  do {                                                                                           \
+    if (cin == 16) SLBN_CONVC(MT, 16);                                                           \
+    else if (cin == 32) SLBN_CONVC(MT, 32);                                                      \
+    else if (cin == 64) SLBN_CONVC(MT, 64);                                                      \
+    else SLBN_CONVC(MT, 0);                                                                      \
+  } while (0)
   if (mt == 1) SLBN_CONV(1);
   else if (mt == 2) SLBN_CONV(2);
   else if (mt == 3) SLBN_CONV(3);
   else if (mt == 4) SLBN_CONV(4);
   else { fprintf(stderr, "slbn_conv: at most 64 output channels\n"); exit(EXIT_FAILURE); }
+#undef SLBN_CONVC
 #undef SLBN_CONV
   LAUNCHCHECK();
 }

@@ -36,6 +36,32 @@ def test_weight_gradient_on_ragged_rows(shape, cin, cout):
     assert np.abs(got[:, :27 * cin] - ref).max() < 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("cin,cout", [(16, 16), (16, 32), (32, 64), (64, 16)])
+@pytest.mark.parametrize("shape", [(4, 4, 64), (16, 128, 64)])   # one, four node tiles per wave
+def test_general_convolution_equals_the_staged_one(shape, cin, cout, monkeypatch):
+    """Same K order and MFMA sequence: bit for bit."""
+    L = lib()
+    rng = np.random.default_rng(cin + cout)
+    xb, _ = bf_random(rng, shape + (cin,))
+    wb, _ = bf_random(rng, (cout, onn.kpad(cin)), 0.1)
+    wb[:, 27 * cin:] = 0
+    dX, dW, n = Dev(host=xb), Dev(host=wb), int(np.prod(shape))
+    got = []
+    for on in "01":
+        monkeypatch.setenv("SLBN_CONV_LDS", on)
+        dY, dF = Dev(n * cout * 2), Dev(n * cout * 4)
+        L.slbn_conv(dX.p, cin, dW.p, None, dY.p, dF.p, cout, 1, 0, *shape)
+        L.slbn_sync()
+        got.append((dY.get(np.uint16, (n, cout)), dF.get(np.uint32, (n, cout))))
+        dY.free()
+        dF.free()
+    dX.free()
+    dW.free()
+    assert got[0][1].any()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("cs,c", [(2, 16), (16, 16), (8, 16), (10, 16), (3, 12), (24, 8)])
 def test_expand(cs, c):
     L = lib()
