@@ -203,10 +203,11 @@ k_bwall_place(const uint16_t *__restrict__ flags, long N, int *__restrict__ plac
   if (x < N) place[x] = has ? base + __popcll(m & ((1ULL << lane) - 1)) : -1;
 }
 
+/* P: the box's first problem; blockIdx.y: its right-hand side, nrow rows each */
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_bwall_fill(const uint16_t *__restrict__ flags, const int32_t *__restrict__ objidx,
-             const int *__restrict__ place, const T *__restrict__ wtab, BProb P,
+             const int *__restrict__ place, const T *__restrict__ wtab, BProb P, int nrow,
              T *__restrict__ rows) {
   const long xl = (long)blockIdx.x * 256 + threadIdx.x;
   if (xl >= P.N) return;
@@ -218,7 +219,8 @@ k_bwall_fill(const uint16_t *__restrict__ flags, const int32_t *__restrict__ obj
   const AxisOff32 oi = axis_off32(i, P.esi, P.plane);
   const AxisOff32 oj = axis_off32(j, P.esj, P.esk);
   const AxisOff32 ok = axis_off32(k, P.esk, 1);
-  T *row = rows + (P.wall_off + place[x]) * 16;
+  const long tab = P.tab_off + (long)blockIdx.y * P.nobj;
+  T *row = rows + (P.wall_off + (long)blockIdx.y * nrow + place[x]) * 16;
   row[14] = row[15] = T(0);
   Links<1, 15>::run([&](auto LL) {
     constexpr int l = decltype(LL)::value;
@@ -231,7 +233,7 @@ k_bwall_fill(const uint16_t *__restrict__ flags, const int32_t *__restrict__ obj
         sj = j - CY(l); sj += (sj < 0) ? P.esj : 0; sj -= (sj >= P.esj) ? P.esj : 0;
         sk = k - CZ(l); sk += (sk < 0) ? P.esk : 0; sk -= (sk >= P.esk) ? P.esk : 0;
       }
-      cu = wall_term<l, T>(wtab + ((long)P.tab_off + objidx[sn]) * WROW, si, sj, sk);
+      cu = wall_term<l, T>(wtab + (tab + objidx[sn]) * WROW, si, sj, sk);
     }
     row[l - 1] = cu;
   });
@@ -639,7 +641,13 @@ static void plan_pairs(slbd_batch *B) {
   free(h);
   /* places of the boxes' boundary nodes, then the moving problems' rows */
   int *cnt, *hc = (int *)calloc(B->nbox, sizeof(int));
-  HIPCHECK(hipMalloc(&B->place, sizeof(int) * B->nnode_tab));
+  if (hipMalloc(&B->place, sizeof(int) * B->nnode_tab) != hipSuccess) {
+    (void)hipGetLastError();
+    B->place = NULL;
+    B->pairs = 0;
+    free(hc);
+    return;
+  }
   HIPCHECK(hipMalloc(&cnt, sizeof(int) * B->nbox));
   HIPCHECK(hipMemsetAsync(cnt, 0, sizeof(int) * B->nbox, B->stream));
   long nrow = 0;
@@ -659,22 +667,35 @@ static void plan_pairs(slbd_batch *B) {
         B->hprobs[B->box_first_prob[b] + r].wall_off = nrow;
         nrow += hc[b];
       }
-  free(hc);
-  HIPCHECK(hipMalloc(&B->wrows, bts(B->prec) * 16 * (nrow > 0 ? nrow : 1)));
-  for (int p = 0; p < B->nprob; p++) {
-    const BProb *q = &B->hprobs[p];
-    if (q->wall_off < 0) continue;
-    const dim3 g((unsigned)((q->N + 255) / 256));
-    if (B->prec == 32)
-      hipLaunchKernelGGL(k_bwall_fill<float>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
-                         B->objidx + q->node_off, B->place + q->node_off, (const float *)B->wtab, *q,
-                         (float *)B->wrows);
-    else
-      hipLaunchKernelGGL(k_bwall_fill<double>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
-                         B->objidx + q->node_off, B->place + q->node_off, (const double *)B->wtab,
-                         *q, (double *)B->wrows);
-    LAUNCHCHECK();
+  /* a batch that fills the memory without the rows runs single steps */
+  if (hipMalloc(&B->wrows, bts(B->prec) * 16 * (nrow > 0 ? nrow : 1)) != hipSuccess) {
+    (void)hipGetLastError();
+    B->wrows = NULL;
+    B->pairs = 0;
+    free(hc);
+    return;
   }
+  for (int b = 0; b < B->nbox; b++) {
+    const BProb *q = &B->hprobs[B->box_first_prob[b]];
+    if (q->wall_off < 0 || hc[b] == 0) continue;
+    BProb q1 = *q;
+    for (int r = 0; r < B->box[b].nrhs; r += 32768) { /* a grid's y extent is 16 bits wide */
+      const int nr = B->box[b].nrhs - r < 32768 ? B->box[b].nrhs - r : 32768;
+      const dim3 g((unsigned)((q->N + 255) / 256), (unsigned)nr);
+      q1.wall_off = q->wall_off + (long)r * hc[b];
+      q1.tab_off = q->tab_off + r * q->nobj;
+      if (B->prec == 32)
+        hipLaunchKernelGGL(k_bwall_fill<float>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
+                           B->objidx + q->node_off, B->place + q->node_off, (const float *)B->wtab,
+                           q1, hc[b], (float *)B->wrows);
+      else
+        hipLaunchKernelGGL(k_bwall_fill<double>, g, dim3(256), 0, B->stream, B->flags + q->node_off,
+                           B->objidx + q->node_off, B->place + q->node_off, (const double *)B->wtab,
+                           q1, hc[b], (double *)B->wrows);
+      LAUNCHCHECK();
+    }
+  }
+  free(hc);
   HIPCHECK(hipStreamSynchronize(B->stream));
 }
 

@@ -152,3 +152,34 @@ def test_batch_pairs_are_single_steps(prec, monkeypatch):
         assert np.all(np.isfinite(a)) and np.array_equal(a, c)
     for a, c in zip(out[0][1], out[1][1]):
         assert np.abs(a - c).max() <= 1e-12 * max(np.abs(a).max(), 1e-30)
+
+
+def test_batch_pairs_many_right_hand_sides(monkeypatch):
+    """More right-hand sides of one box than a launch of the wall rows takes
+    (32768): populations of the problems at that edge, bit for bit."""
+    import sunlightlb_amd as s
+    nrhs, out = 32770, []
+    for on in "01":
+        monkeypatch.setenv("SLB_BATCH_STEP2", on)
+        print(f"batch pairs: {nrhs} right-hand sides, pairs {on}", flush=True)
+        lat = s.Lattice(6, 5, 4, precision=32)
+        L = lat.L
+        lat.s.tau, lat.s.stokes_flow, lat.s.objects_moving = 0.7, 1, 1
+        assert L.insertsph(lat.h, 1.3, 2.6, 2.2, 1.7)
+        n = len(lat.objects())
+        vel = np.random.default_rng(3).normal(0, 0.01, (nrhs, n, 6))
+        b = L.slb_batch_new(32)
+        assert L.slb_batch_add(b, lat.h, nrhs, vel.ctypes.data_as(C.POINTER(C.c_double))) == 0
+        lat.free()
+        assert L.slb_batch_commit(b) == 0
+        L.slb_batch_run(b, 4)
+        got = []
+        for r in (0, 1, 32767, 32768, 32769):
+            a = np.zeros(15 * 120)
+            L.slb_batch_get_pops(b, 0, r, a.ctypes.data_as(C.POINTER(C.c_double)))
+            assert np.abs(a).max() > 1e-6
+            got.append(a)
+        out.append(got)
+        L.slb_batch_free(b)
+    for a, c in zip(*out):
+        assert np.array_equal(a, c)
