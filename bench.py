@@ -221,15 +221,16 @@ def cpu_batch_baseline(boxes, steps, u0, tau, nbox=16, per_proc=8, max_procs=16)
     return res
 
 
-def traffic_bytes(n, precision):
-    """HBM bytes per k_step launch measured by rocprofv3 --pmc FETCH_SIZE and
-    WRITE_SIZE on this workload, each scaled by the factor the same counter
-    reads for a plain copy of known size (profiles/k_step_traffic.json)."""
+def traffic_bytes(n, precision, pairs):
+    """HBM bytes per step (a k_step2 launch is two steps) measured by rocprofv3
+    --pmc FETCH_SIZE and WRITE_SIZE on this workload, each scaled by the
+    factor the same counter reads for a plain copy of known size
+    (profiles/k_step_traffic.json)."""
     path = os.path.join(ROOT, "profiles", "k_step_traffic.json")
     try:
         with open(path) as f:
             t = json.load(f)
-        key = f"{n}_fp{precision}"
+        key = f"{n}_fp{precision}" + ("_pairs" if pairs else "")
         return t["workloads"][key]["traffic_bytes"] if key in t["workloads"] else None
     except (OSError, KeyError, ValueError):
         return None
@@ -307,8 +308,10 @@ def mp_run(L, args, prec, n, R, phi, peclet, alpha, pads, baseline):
     mlups = N * args.mp_steps / (ms * 1e-3) / 1e6
     # algorithmic bytes: the 15 link factors of a node (from its 15 pulled
     # populations of the frozen flow, precomputed once per run) and the node's
-    # {P, m1, m2} read and written
-    bpl = (15 + 2 * 3) * (4 if prec == 32 else 8)
+    # {P, m1, m2} read and written, once for two steps where the run pairs them
+    ts = 4 if prec == 32 else 8
+    pairs = 15 * N * ts >= 36e6 and os.environ.get("SLB_MP_STEP2", "1") != "0"
+    bpl = (15 + 2 * 3) * ts / (2 if pairs else 1)
     res = {
         "workload": f"{n}^3 RSA pack R {R:g} phi {phi_got:.4f} ({nsph} spheres), flow solved "
                     f"to residual {r.value:.2e} in {steps} steps, scaled to Pe {peclet:g} "
@@ -483,7 +486,9 @@ def batch_run(L, args, prec, boxes, u0, tau, tune):
     ms = L.slb_batch_time_steps(b, args.batch_steps)
     L.slb_batch_measure(b)
     mlups = nodes * args.batch_steps / (ms * 1e-3) / 1e6
-    bpl = 2 * 15 * (4 if prec == 32 else 8)
+    # one read and one write of the populations per two steps (k_bstep2)
+    pairs = os.environ.get("SLB_BATCH_STEP2", "1") != "0"
+    bpl = (1 if pairs else 2) * 15 * (4 if prec == 32 else 8)
     mats = resistance_matrices(L, b, moving_rows, u0)
     L.slb_batch_free(b)
     res = {
@@ -960,7 +965,7 @@ def main():
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",
             "frac": round(achieved / PEAK_HBM_GBS, 4),
-            "traffic": traffic_bytes(n, args.precision),
+            "traffic": traffic_bytes(n, args.precision, pairs),
             # the kernel the library launches for this lattice's steps
             "kernel": kernel + {"k_step2": " (two fused pull steps per pass)",
                                 "k_step_lds": " (fused pull step, k pulls staged in LDS)",

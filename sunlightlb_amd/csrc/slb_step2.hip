@@ -16,8 +16,9 @@
  *     (both wait in registers); the tile's nodes collide again and are
  *     written.
  *
- * Bound by HBM and its latency at 256^3 (2.3 GB for two steps, 77% of the
- * copy rate; the VALU is busy 42% of the time).  Measured, us per step, one
+ * Bound by HBM and its latency at 256^3: FP32 2.36 GB for two steps (1.17x
+ * one read and one write), 80% of the copy rate, the VALU busy 40% of the
+ * time; FP64 4.82 GB, 98%, 29%.  Measured, us per step, one
  * step at a time / this kernel: FP32 256^3 356.6/224.0, 512^3 2957/1852,
  * 160^3 94.4/58.8, 96^3 20.7/12.6, 64^3 6.97/6.05; FP64 256^3 735/401,
  * 128^3 92.9/54.7, 32^3 5.69/3.87.
