@@ -1406,7 +1406,7 @@ struct slbd_lattice {
   int sweep_nt_mid;         /* two-step sweep: non-temporal window stores */
   int step_lds;             /* step with the k pulls staged in LDS (k_step_lds) */
   int ldsr_rpb, ldsr_bs;    /* k_step_ldsr: rows per block, threads per block (0: off) */
-  int pairs, pair_nt;       /* runs take their steps two at a time (k_step2); its store hint */
+  int pairs, pair_nt, pair_mode; /* runs take their steps two at a time (k_step2); its store hint, addressing */
   Step2Plan plan2;
   void *mom[2];             /* moment storage of a run (k_step_mom), or NULL */
   void *sph_buf;            /* sphere images of a pack being placed (grow-only) */
@@ -1478,8 +1478,8 @@ extern "C" const char *slbd_arch(void) {
 /* Whether runs with walls at rest take their steps two at a time (k_step2):
  * always, since it is the faster one on every shape measured
  * (slb_step2.hip), unless SLB_STEP2=0
- * or the environment names a single-step kernel or 64-bit indices.  Lattices
- * beyond 32-bit population indices need planes of whole population tiles.
+ * or the environment names a single-step kernel or 64-bit indices, or no
+ * addressing of k_step2 reaches the lattice (slbd_step2_mode).
  * Stores are non-temporal except where both buffers fit the 256 MB last-level
  * cache and exceed the L2s by far, and the next pass reads them there, and
  * where rows start off a 128-byte line, and two tiles share its lines: nt /
@@ -1490,8 +1490,9 @@ static void pair_policy(slbd_lattice *L) {
   const long np = 15 * pop_nodes(L->N), ts = (long)tsize(L->prec);
   const char *e = getenv("SLB_STEP2");
   const bool small = np <= 0x7fffffffL;
+  L->pair_mode = slbd_step2_mode(L->G.plane, L->N, L->prec);
   L->pairs = !(e && atoi(e) == 0) && !getenv("SLB_STEP_LDS") && L->idx32 == (int)small &&
-             (small || (L->G.plane % POP_TILE == 0 && 15L * L->G.plane * ts < (1L << 32))) &&
+             L->pair_mode >= 0 &&
              slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2);
   const double both = 30.0 * (double)L->N * (double)ts;
   const bool lines = ((long)L->esk * ts) % 128 == 0 &&
@@ -2295,7 +2296,7 @@ extern "C" void slbd_step(slbd_lattice *L, const slbd_params *P, int nsteps, int
   if (L->pairs && sw == 0 && !force && !P->moving)
     for (; s + 2 <= nsteps; s += 2) {
       const Step2Args a = {L->pops[L->cur], L->pops[L->cur ^ 1], L->flags, L->bx, L->by, L->bz,
-                           L->pair_nt != 0, bf, L->plan2};
+                           L->pair_nt != 0, bf, L->pair_mode, L->plan2};
       slbd_step2_launch(&a, A, L->G, L->prec, L->stream);
       L->cur ^= 1;
     }

@@ -42,13 +42,25 @@ struct Step2Plan {
  * which three waves per SIMD fit). */
 template <typename T> struct Step2Cfg { enum { NTHR = sizeof(T) == 4 ? 1024 : 768 }; };
 
+/* How a column's accesses are addressed: the first of these that
+ * slbd_step2_mode_ok allows.
+ * 0: planes of whole population tiles (plane % 1024 == 0) and buffers under
+ *    4 GB: a column's in-plane byte offset is fixed and a plane adds a scalar;
+ * 1: any plane, buffers under 4 GB (two more operations per load);
+ * 2: as 0 with 64-bit plane offsets: the in-plane byte offset has 32 bits, so
+ *    planes are under 4 GB (a lattice of few planes can exceed that while its
+ *    population indices still have 31 bits);
+ * 3: any plane, 31-bit population indices. */
+extern "C" int slbd_step2_mode_ok(int mode, long plane, long N, int prec);
+extern "C" int slbd_step2_mode(long plane, long N, int prec);   /* -1: none */
+
 struct Step2Args {
   const void *src;
   void *dst;
   const uint16_t *flags;
   const void *bx, *by, *bz;
   bool nt;
-  int bf;
+  int bf, mode;
   Step2Plan plan;
 };
 

@@ -40,11 +40,7 @@
 #include "slb_kern.h"
 #include "slb_step2.h"
 
-/* MODE 0: planes of whole population tiles (plane % 1024 == 0) and buffers
- * under 4 GB: a column's in-plane byte offset is fixed and a plane adds a
- * scalar; MODE 1: any plane, buffers under 4 GB (two more operations per
- * load); MODE 2: as 0 with 64-bit plane offsets; MODE 3: any plane, 32-bit
- * population indices.  NT: non-temporal stores. */
+/* MODE: slbd_step2_mode.  NT: non-temporal stores. */
 template <typename T, int BF, int MODE, bool NT>
 __global__ void __launch_bounds__(Step2Cfg<T>::NTHR)
 k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restrict__ flags,
@@ -274,6 +270,24 @@ int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best) {
   return best->ci > 0;
 }
 
+extern "C" int slbd_step2_mode_ok(int mode, long plane, long N, int prec) {
+  const long ts = prec == 32 ? 4 : 8, four = 1L << 32, np = 15 * pop_nodes(N);
+  const bool whole = plane % POP_TILE == 0;
+  switch (mode) {
+    case 0: return whole && np * ts < four;
+    case 1: return np * ts < four;
+    case 2: return whole && 15 * plane * ts < four;
+    case 3: return np <= 0x7fffffffL;
+    default: return 0;
+  }
+}
+
+extern "C" int slbd_step2_mode(long plane, long N, int prec) {
+  for (int m = 0; m < 4; m++)
+    if (slbd_step2_mode_ok(m, plane, N, prec)) return m;
+  return -1;
+}
+
 template <typename T, int MODE, bool NT>
 static void launch2(const Step2Args *a, const PhysArgs &A, const Geom &G, hipStream_t st) {
   const int pts = (a->plan.jt + 2) * (a->plan.kt + 2);
@@ -297,14 +311,16 @@ static void launch2(const Step2Args *a, const PhysArgs &A, const Geom &G, hipStr
 
 template <typename T>
 static void launch2_t(const Step2Args *a, const PhysArgs &A, const Geom &G, hipStream_t st) {
-  const bool whole = G.plane % POP_TILE == 0;
-  const bool small = 15 * pop_nodes(G.N) * (long)sizeof(T) < (1L << 32);
-  if (whole && small) {
+  if (!slbd_step2_mode_ok(a->mode, G.plane, G.N, (int)sizeof(T) * 8)) {
+    fprintf(stderr, "sunlightlb: a two-step pass cannot address this lattice in mode %d\n", a->mode);
+    exit(EXIT_FAILURE);
+  }
+  if (a->mode == 0) {
     if (a->nt) launch2<T, 0, true>(a, A, G, st); else launch2<T, 0, false>(a, A, G, st);
-  } else if (whole) {
-    launch2<T, 2, true>(a, A, G, st);
-  } else if (small) {
+  } else if (a->mode == 1) {
     if (a->nt) launch2<T, 1, true>(a, A, G, st); else launch2<T, 1, false>(a, A, G, st);
+  } else if (a->mode == 2) {
+    launch2<T, 2, true>(a, A, G, st);
   } else {
     launch2<T, 3, true>(a, A, G, st);
   }
