@@ -1485,12 +1485,16 @@ extern "C" const char *slbd_arch(void) {
  * where rows start off a 128-byte line, and two tiles share its lines: nt /
  * plain us per FP32 step at 96^3 (106 MB) 15.8/12.6, 128^3 (252 MB)
  * 31.9/30.4, 160^3 (491 MB) 58.8/61.5, 64^3 (31 MB) 6.05/6.31; off the line
- * 200^3 152/141, 400^3 1519/1258. */
+ * 200^3 152/141, 400^3 1519/1258, 420^3 1148/1130 (FP64 340^3 1317/1159). */
 static void pair_policy(slbd_lattice *L) {
   const long np = 15 * pop_nodes(L->N), ts = (long)tsize(L->prec);
   const char *e = getenv("SLB_STEP2");
   const bool small = np <= 0x7fffffffL;
   L->pair_mode = slbd_step2_mode(L->G.plane, L->N, L->prec);
+  if (getenv("SLB_STEP2_MODE")) {      /* another one that reaches the lattice (tests) */
+    const int m = atoi(getenv("SLB_STEP2_MODE"));
+    if (slbd_step2_mode_ok(m, L->G.plane, L->N, L->prec)) L->pair_mode = m;
+  }
   L->pairs = !(e && atoi(e) == 0) && !getenv("SLB_STEP_LDS") && L->idx32 == (int)small &&
              L->pair_mode >= 0 &&
              slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2);

@@ -320,9 +320,9 @@ static void launch2_t(const Step2Args *a, const PhysArgs &A, const Geom &G, hipS
   } else if (a->mode == 1) {
     if (a->nt) launch2<T, 1, true>(a, A, G, st); else launch2<T, 1, false>(a, A, G, st);
   } else if (a->mode == 2) {
-    launch2<T, 2, true>(a, A, G, st);
+    if (a->nt) launch2<T, 2, true>(a, A, G, st); else launch2<T, 2, false>(a, A, G, st);
   } else {
-    launch2<T, 3, true>(a, A, G, st);
+    if (a->nt) launch2<T, 3, true>(a, A, G, st); else launch2<T, 3, false>(a, A, G, st);
   }
 }
 

@@ -183,3 +183,35 @@ def test_batch_pairs_many_right_hand_sides(monkeypatch):
         L.slb_batch_free(b)
     for a, c in zip(*out):
         assert np.array_equal(a, c)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("dims,stokes,skip,bf,nt", [
+    ((9, 32, 64), 0, 1, 2, 1),        # whole tiles per plane, per-node body force
+    ((1, 32, 32), 1, 0, 1, 0),        # one plane, a neighbour of itself
+    ((5, 8, 512), 1, 1, 0, 1),        # more than one k tile, no body force
+    ((4, 11, 331), 0, 0, 1, 1),       # k tiles of unequal width; rows off the 128-byte lines
+    ((1, 1, 7), 0, 0, 1, 0), ((3, 2, 1), 1, 1, 2, 1),
+])
+def test_every_addressing_mode_is_single_steps(dims, stokes, skip, bf, nt, mode, prec, monkeypatch):
+    """The addressing of buffers over 4 GB (modes 2 and 3) on small lattices:
+    every mode that reaches the lattice, with and without non-temporal stores."""
+    import sunlightlb_amd as s
+    L = s.lib()
+    L.slbd_step2_mode_ok.argtypes = [C.c_int, C.c_long, C.c_long, C.c_int]
+    plane = dims[1] * dims[2]
+    if not L.slbd_step2_mode_ok(mode, plane, dims[0] * plane, prec):
+        assert mode in (0, 2) and plane % 1024
+        return
+    print(f"pairs: {dims} prec {prec} mode {mode} nt {nt}", flush=True)
+    monkeypatch.setenv("SLB_STEP2_MODE", str(mode))
+    monkeypatch.setenv("SLB_NT_STORE", str(nt))
+    ref, got = (build(dims, prec, 0, stokes, skip, bf) for _ in range(2))
+    for n in (2, 5):
+        for _ in range(n):
+            ref.L.lbstep(ref.h)
+        got.L.slb_run(got.h, n)
+        assert np.array_equal(ref.pops(), got.pops())
+    ref.free()
+    got.free()
