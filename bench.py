@@ -310,7 +310,7 @@ def mp_run(L, args, prec, n, R, phi, peclet, alpha, pads, baseline):
     # populations of the frozen flow, precomputed once per run) and the node's
     # {P, m1, m2} read and written, once for two steps where the run pairs them
     ts = 4 if prec == 32 else 8
-    pairs = 15 * N * ts >= 36e6 and os.environ.get("SLB_MP_STEP2", "1") != "0"
+    pairs = L.slb_mp_run_kernel(mp, args.mp_steps) == b"k_mpstep2"
     bpl = (15 + 2 * 3) * ts / (2 if pairs else 1)
     res = {
         "workload": f"{n}^3 RSA pack R {R:g} phi {phi_got:.4f} ({nsph} spheres), flow solved "
@@ -487,7 +487,7 @@ def batch_run(L, args, prec, boxes, u0, tau, tune):
     L.slb_batch_measure(b)
     mlups = nodes * args.batch_steps / (ms * 1e-3) / 1e6
     # one read and one write of the populations per two steps (k_bstep2)
-    pairs = os.environ.get("SLB_BATCH_STEP2", "1") != "0"
+    pairs = L.slb_batch_run_kernel(b) == b"k_bstep2"
     bpl = (1 if pairs else 2) * 15 * (4 if prec == 32 else 8)
     mats = resistance_matrices(L, b, moving_rows, u0)
     L.slb_batch_free(b)
@@ -915,11 +915,10 @@ def main():
     h, nsph, phi = build_pack(L, n, args.radius, args.phi, args.seed, args.force)
     N = n ** 3
 
-    # runs with walls at rest take two steps per pass over the populations
-    # (k_step2), one read and one write for both, unless the environment
-    # names a single-step kernel
-    pairs = os.environ.get("SLB_STEP2", "1") != "0" and "SLB_STEP_LDS" not in os.environ
-    kernel = "k_step2" if pairs else L.slb_step_kernel(h).decode()
+    # where runs take two steps per pass over the populations (k_step2), one
+    # read and one write serve both
+    kernel = L.slb_run_kernel(h).decode()
+    pairs = kernel == "k_step2"
     L.slb_run(h, args.warmup)
     ms = L.slb_time_steps(h, args.steps)
     ms_per_step = ms / args.steps

@@ -81,6 +81,11 @@ double slb_time_steps(LBSys lb, int nsteps);
  * step, SLB_STEP2=0 keeps runs to single steps. */
 const char *slb_step_kernel(LBSys lb);
 
+/* Name of the kernel that slb_run's steps launch as the lattice stands now
+ * (walls at rest or moving, environment): "k_step2" where they go two per pass
+ * (an odd last one is slb_step_kernel's), "k_step_mom", or slb_step_kernel's. */
+const char *slb_run_kernel(LBSys lb);
+
 /* Multiply every population by s (a Stokes-flow solution scales with the
  * body force). */
 void slb_scale_pops(LBSys lb, double s);
@@ -153,6 +158,10 @@ void slb_mp_sums(MPSys mp, double out[6]);
  * always), with the same results. */
 void slb_mp_run(MPSys mp, int nsteps);
 
+/* Name of the kernel that slb_mp_run(mp, nsteps) launches: "k_mpstep2" (two
+ * steps per pass), "k_mpstep_w" (precomputed link factors) or "k_mpstep". */
+const char *slb_mp_run_kernel(MPSys mp, int nsteps);
+
 /* Time nsteps MP steps on the device between HIP events (the state
  * advances).  Returns milliseconds. */
 double slb_mp_time_steps(MPSys mp, int nsteps);
@@ -191,6 +200,9 @@ void slb_batch_set_config(SLBBatch b, int block, int nodes_per_thread, int grid)
 void slb_batch_get_config(SLBBatch b, int cfg[4]);
 
 void   slb_batch_run(SLBBatch b, int nsteps);
+/* Name of the kernel that a committed batch's runs launch: "k_bstep2" (two
+ * steps per pass; an odd last step is k_bstep's) or "k_bstep". */
+const char *slb_batch_run_kernel(SLBBatch b);
 double slb_batch_time_steps(SLBBatch b, int nsteps);
 /* measure(): two force-collecting steps, force and torque per object halved
  * (FP64 sums, torque about each object's own centre, no minimum image). */

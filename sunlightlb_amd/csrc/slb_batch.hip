@@ -895,6 +895,10 @@ extern "C" void slbd_batch_run(slbd_batch *B, int nsteps, int use_graph) {
   bsteps(B, nsteps - s, B->pairs != 0 && use_graph != 0);
 }
 
+extern "C" const char *slbd_batch_run_kernel(const slbd_batch *B) {
+  return B->committed && B->pairs ? "k_bstep2" : "k_bstep";
+}
+
 extern "C" double slbd_batch_time(slbd_batch *B, int nsteps, int use_graph) {
   if (use_graph && B->committed && nsteps >= BATCH_GRAPH_STEPS) build_graph(B);
   HIPCHECK(hipStreamSynchronize(B->stream));

@@ -137,6 +137,8 @@ void slb_batch_run(SLBBatch b, int nsteps) {
   slbd_batch_run(b->d, nsteps, 1);
 }
 
+const char *slb_batch_run_kernel(SLBBatch b) { return slbd_batch_run_kernel(b->d); }
+
 double slb_batch_time_steps(SLBBatch b, int nsteps) {
   b->stepped = 1;
   return slbd_batch_time(b->d, nsteps, 1);

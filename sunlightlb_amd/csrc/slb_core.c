@@ -808,6 +808,12 @@ int slb_run_to_residual_aa(LBSys lb, double tol, int interval, int maxsteps, int
 
 const char *slb_step_kernel(LBSys lb) { return slbd_step_kernel(PRIV(lb)->dev); }
 
+const char *slb_run_kernel(LBSys lb) {
+  slbd_params P;
+  slb_params(lb, &P);
+  return slbd_run_kernel(PRIV(lb)->dev, &P);
+}
+
 double slb_time_steps(LBSys lb, int nsteps) {
   if (lb->changed_objects) syncobjs(lb);
   slbd_params P;

@@ -150,8 +150,10 @@ void slbd_vacf(slbd_lattice *L, slbd_mp *M, slbd_mp *M2, const double *psi_host,
  * lattice stream; returns the elapsed milliseconds. */
 double slbd_time_steps(slbd_lattice *L, const slbd_params *P, int nsteps);
 const char *slbd_step_kernel(const slbd_lattice *L);
+const char *slbd_run_kernel(const slbd_lattice *L, const slbd_params *P);
 double slbd_time_mp(slbd_lattice *L, slbd_mp *M, double rho0, double alpha,
                     double pads, int nmom, int nsteps);
+const char *slbd_mp_run_kernel(const slbd_lattice *L, slbd_mp *M, int nsteps);
 size_t slbd_bytes(const slbd_lattice *L);
 /* Plain 16-byte-per-lane copy of `bytes` between two device buffers, reps
  * times; mean milliseconds per copy (HBM roofline and counter calibration). */
@@ -223,6 +225,7 @@ void slbd_batch_config(slbd_batch *B, int block, int npt, int grid);
 void slbd_batch_get_config(const slbd_batch *B, int *cfg);
 void slbd_batch_run(slbd_batch *B, int nsteps, int use_graph);
 double slbd_batch_time(slbd_batch *B, int nsteps, int use_graph);
+const char *slbd_batch_run_kernel(const slbd_batch *B);
 void slbd_batch_measure(slbd_batch *B);
 int  slbd_batch_forces(slbd_batch *B, int box, int rhs, double *frc, double *trq);
 int  slbd_batch_get_pops(slbd_batch *B, int box, int rhs, double *aos);

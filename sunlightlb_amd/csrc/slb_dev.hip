@@ -2280,6 +2280,10 @@ static void mom_run(slbd_lattice *L, const PhysArgs &A, bool moving, int bf, int
   L->cur ^= 1;
 }
 
+static bool takes_pairs(const slbd_lattice *L, const slbd_params *P, int sweep) {
+  return L->pairs && sweep == 0 && !P->moving;
+}
+
 extern "C" void slbd_step(slbd_lattice *L, const slbd_params *P, int nsteps, int force) {
   const PhysArgs A = phys(P);
   const int bf = bf_mode(L, P);
@@ -2297,7 +2301,7 @@ extern "C" void slbd_step(slbd_lattice *L, const slbd_params *P, int nsteps, int
       else sweep2<double>(L, A, P->moving != 0, bf, sw);
     }
   }
-  if (L->pairs && sw == 0 && !force && !P->moving)
+  if (!force && takes_pairs(L, P, sw))
     for (; s + 2 <= nsteps; s += 2) {
       const Step2Args a = {L->pops[L->cur], L->pops[L->cur ^ 1], L->flags, L->bx, L->by, L->bz,
                            L->pair_nt != 0, bf, L->pair_mode, L->plan2};
@@ -2319,6 +2323,13 @@ extern "C" const char *slbd_step_kernel(const slbd_lattice *L) {
   if (L->step_lds) return "k_step_lds";
   if (L->ldsr_rpb) return "k_step_ldsr";
   return "k_step";
+}
+
+/* Name of the kernel that a run's steps launch. */
+extern "C" const char *slbd_run_kernel(const slbd_lattice *L, const slbd_params *P) {
+  const int sw = sweep_planes(L);
+  if (sw == 0 && mom_run_ok(L, P, 2, 0)) return "k_step_mom";
+  return takes_pairs(L, P, sw) ? "k_step2" : slbd_step_kernel(L);
 }
 
 extern "C" double slbd_time_steps(slbd_lattice *L, const slbd_params *P, int nsteps) {
@@ -2806,6 +2817,13 @@ extern "C" void slbd_mp_step(slbd_lattice *L, slbd_mp *M, double rho0, double al
   A.rho0 = rho0; A.alpha = alpha; A.pads = pads; A.axis = axis;
   if (L->prec == 32) launch_mp<float>(L, M, A, moving != 0, nsteps);
   else launch_mp<double>(L, M, A, moving != 0, nsteps);
+}
+
+/* Name of the kernel that a run of nsteps MP steps launches. */
+extern "C" const char *slbd_mp_run_kernel(const slbd_lattice *L, slbd_mp *M, int nsteps) {
+  const int wmin = mp_weights_min();
+  if (wmin <= 0 || nsteps < wmin) return "k_mpstep";
+  return mp_pairs(L, M) ? "k_mpstep2" : "k_mpstep_w";
 }
 
 extern "C" double slbd_time_mp(slbd_lattice *L, slbd_mp *M, double rho0, double alpha,

@@ -144,6 +144,10 @@ void slb_mp_run(MPSys mp, int nsteps) {
   mp->step += nsteps;
 }
 
+const char *slb_mp_run_kernel(MPSys mp, int nsteps) {
+  return slbd_mp_run_kernel(PRIV(mp->lb)->dev, MPRIV(mp)->dev, nsteps);
+}
+
 double slb_mp_time_steps(MPSys mp, int nsteps) {
   slb_mppriv *M = MPRIV(mp);
   LBSys lb = mp->lb;
