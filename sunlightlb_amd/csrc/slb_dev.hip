@@ -1476,10 +1476,10 @@ extern "C" const char *slbd_arch(void) {
 }
 
 /* Whether runs with walls at rest take their steps two at a time (k_step2):
- * always, since it is the faster one on every shape measured
- * (slb_step2.hip), unless SLB_STEP2=0
- * or the environment names a single-step kernel or 64-bit indices, or no
- * addressing of k_step2 reaches the lattice (slbd_step2_mode).
+ * where it is the faster way (slbd_step2_pays; SLB_STEP2=1 wherever a tile
+ * fits), unless SLB_STEP2=0 or the environment names a single-step kernel or
+ * 64-bit indices, or no addressing of k_step2 reaches the lattice
+ * (slbd_step2_mode).
  * Stores are non-temporal except where both buffers fit the 256 MB last-level
  * cache and exceed the L2s by far, and the next pass reads them there, and
  * where rows start off a 128-byte line, and two tiles share its lines: nt /
@@ -1497,7 +1497,8 @@ static void pair_policy(slbd_lattice *L) {
   }
   L->pairs = !(e && atoi(e) == 0) && !getenv("SLB_STEP_LDS") && L->idx32 == (int)small &&
              L->pair_mode >= 0 &&
-             slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2);
+             slbd_step2_plan(L->esi, L->esj, L->esk, L->prec, &L->plan2) &&
+             (e || slbd_step2_pays(L->esi, L->esj, L->esk, L->prec, &L->plan2));
   const double both = 30.0 * (double)L->N * (double)ts;
   const bool lines = ((long)L->esk * ts) % 128 == 0 &&
                      (L->plan2.nkt == 1 || ((long)L->plan2.kt * ts) % 128 == 0);

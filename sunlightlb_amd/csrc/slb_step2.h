@@ -64,7 +64,8 @@ struct Step2Args {
   Step2Plan plan;
 };
 
-int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best);
+extern "C" int slbd_step2_pays(int esi, int esj, int esk, int prec, const Step2Plan *p);
+extern "C" int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best);
 void slbd_step2_launch(const Step2Args *a, const PhysArgs &A, const Geom &G, int prec,
                        hipStream_t st);
 

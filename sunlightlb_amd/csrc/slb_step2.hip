@@ -241,8 +241,10 @@ k_step2(const T *__restrict__ src, T *__restrict__ dst, const uint16_t *__restri
  * nodes and a constant for the barrier and the load latency (1000 nodes, from
  * tiles of 13 x 64 and 8 x 64 nodes at 256^3).  Short rows cost more (FP32
  * 256^3: 4 x 128 tiles 224 us per step, 13 x 64 232, 26 x 32 270), and so do
- * rows that start off a 128-byte line (FP64 256^3: 84 x 9 509, 64 x 8 401). */
-int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best) {
+ * rows that start off a 128-byte line (FP64 256^3: 84 x 9 509, 64 x 8 401), which
+ * those of a lattice with such rows do whatever the tile's width (FP32 20 x 109 x
+ * 665: 28 x 32 tiles 34.6, 7 x 84 17.6). */
+extern "C" int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best) {
   const int cap = prec == 32 ? Step2Cfg<float>::NTHR : Step2Cfg<double>::NTHR;
   const int cus = 256, wide = prec == 32 ? 160 : 100;
   double bc = 0.0;
@@ -250,7 +252,8 @@ int slbd_step2_plan(int esi, int esj, int esk, int prec, Step2Plan *best) {
   for (int nk = (esk + wide - 1) / wide; nk <= (esk + 31) / 32; nk++) {
     const int kt = (esk + nk - 1) / nk, nkt = (esk + kt - 1) / kt;
     const int jmax = cap / (kt + 2) - 2;
-    const double row = (1.0 + 16.0 / kt) * (nkt > 1 && (long)kt * (prec / 8) % 128 ? 1.2 : 1.0);
+    const bool line = (long)kt * (prec / 8) % 128 == 0 && (long)esk * (prec / 8) % 128 == 0;
+    const double row = (1.0 + 16.0 / kt) * (nkt > 1 && !line ? 1.2 : 1.0);
     for (int jq = 1; jq <= jmax && jq <= esj; jq++) {
       const int njt = (esj + jq - 1) / jq, jt = (esj + njt - 1) / njt;
       for (int r = 1; r <= 3; r++) {     /* as many chunks as r rounds hold */
@@ -286,6 +289,34 @@ extern "C" int slbd_step2_mode(long plane, long N, int prec) {
   for (int m = 0; m < 4; m++)
     if (slbd_step2_mode_ok(m, plane, N, prec)) return m;
   return -1;
+}
+
+/* Whether two steps per pass are the faster way on the tiles of plan p.  A
+ * block computes step t+1 on a rim around its tile and on the planes before
+ * and after its chunk: `work` nodes per node of the result.  Not
+ *   - in several rounds of blocks with a work of more than 3.2, as a single
+ *     plane of a large lattice has (three planes marched for one): single / two
+ *     steps per pass, us per FP32 step, 1 x 1024 x 1024 19/23, 1 x 2923 x 899
+ *     54/65, 1 x 1 x 65536 3.9/5.1 (FP64 36/41, 1 x 759 x 2191 77/91, 4.8/8.6);
+ *     but 2 x 1024 x 1024 (2.4) 36/32 (FP64 97/60), 1236 x 1 x 2635 in one round
+ *     (3.1) 89/67, 1 x 256 x 256 4.6/3.5;
+ *   - on long chunks of planes of up to 160 nodes (FP64 80), a march of a barrier
+ *     and a load latency each for next to nothing (1.0-1.4 us per plane): 65536 x 1 x 1
+ *     42/140, 4096 x 1 x 1 5.8/10.8, 1671 x 12 x 2 5.2/6.1, 5000 x 8 x 8 9.2/14.9 (FP64
+ *     13/17), 12000 x 10 x 10 27.7/31.5; but FP64 12000 x 10 x 10 55/43, and in
+ *     chunks of 4 planes 1000 x 10 x 10 6.3/5.3;
+ *   - on a few long rows, which are split over k into tiles of mostly rim:
+ *     3 x 8 x 2034 3.8/4.7, 7 x 7 x 1294 5.0/5.2.
+ * Elsewhere it is faster or, within the spread of two runs of such calls,
+ * equal (380 shapes with one to three short axes, 64 to 16 million nodes, both
+ * precisions: 0.5-0.9 of the time, a few of 20-100 thousand nodes 1.0-1.1). */
+extern "C" int slbd_step2_pays(int esi, int esj, int esk, int prec, const Step2Plan *p) {
+  const double work = (p->jt + 2.0) * (p->kt + 2.0) * (p->ci + 2.0) / ((double)p->jt * p->kt * p->ci);
+  const long blocks = (long)p->njt * p->nkt * p->nch, plane = (long)esj * esk;
+  if (blocks > 256 && work > 3.2) return 0;
+  if (plane * (prec / 8) <= 640 && p->ci > 6) return 0;
+  if (esk > 1000 && work > 5.0 && esi * plane > 8192) return 0;
+  return 1;
 }
 
 template <typename T, int MODE, bool NT>
