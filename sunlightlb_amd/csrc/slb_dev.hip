@@ -2710,8 +2710,9 @@ static int mp_weights_min(void) {
  * Single / paired, us per FP32 step with moments: 64^3 (16 MB of factors)
  * 4.7/5.9, 80^3 (31 MB) 8.8/9.7, 100 x 90 x 70 (38 MB) 12.5/10.8, 128^3
  * 26.5/19.7, 256^3 322/153; FP64: 64^3 (31 MB) 10.3/11.4, 120 x 61 x 45 (40 MB)
- * 12.9/11.3, 128^3 78.7/44.2.  SLB_MP_STEP2=0 never, =1 wherever a tile fits
- * (read per call). */
+ * 12.9/11.3, 128^3 78.7/44.2.  Of the larger ones, where the tiles are not mostly
+ * rim (slbd_mp2_pays).  SLB_MP_STEP2=0 never, =1 wherever a tile fits (read per
+ * call). */
 static bool mp_pairs(const slbd_lattice *L, slbd_mp *M) {
   const char *e = getenv("SLB_MP_STEP2");
   const bool large = 15.0 * (double)L->N * (double)tsize(L->prec) >= 36e6;
@@ -2720,7 +2721,7 @@ static bool mp_pairs(const slbd_lattice *L, slbd_mp *M) {
     M->planned = 1;
     slbd_mp2_plan(L->esi, L->esj, L->esk, L->prec, M->nmom, &M->plan2);
   }
-  return M->plan2.ci > 0;
+  return M->plan2.ci > 0 && (e || slbd_mp2_pays(L->esj, L->esk, M->nmom, &M->plan2));
 }
 
 template <typename T, int NMOM, bool MOVING>

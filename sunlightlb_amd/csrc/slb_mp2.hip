@@ -187,7 +187,7 @@ k_mpstep2(const T *__restrict__ wt, const CRec<T, NMOM> *__restrict__ Q,
 /* Tiles: as slbd_step2_plan, the split of least cost over rounds of blocks,
  * with the same weights for short and unaligned rows (128^3 FP32: 13 x 64 19.6
  * us per step, 5 x 128 23.6, 26 x 26 27.2). */
-int slbd_mp2_plan(int esi, int esj, int esk, int prec, int nmom, MP2Plan *best) {
+extern "C" int slbd_mp2_plan(int esi, int esj, int esk, int prec, int nmom, MP2Plan *best) {
   const int cap = prec == 32 ? MP2Cfg<float>::NTHR : MP2Cfg<double>::NTHR;
   const long rec = (long)(prec / 8) * (nmom > 1 ? 3 : 1);
   const int cus = 256;
@@ -219,6 +219,29 @@ int slbd_mp2_plan(int esi, int esj, int esk, int prec, int nmom, MP2Plan *best) 
     }
   }
   return best->ci > 0;
+}
+
+/* Whether two steps per pass are the faster way on the tiles of plan p, given
+ * factors beyond the L2s.  `work`: nodes of step t+1 per node of the result,
+ * the rim and the planes before and after a chunk included.  Not
+ *   - with a work of more than 3.3 (one moment 3.5): single / two steps per
+ *     pass, us per step with moments, FP32 1 x 1024 x 1024 14/23, 1 x 2923 x 899
+ *     40/62, 1024 x 1024 x 1 14/17.5, FP64 1 x 2907 x 2023 196/270; one moment FP32
+ *     1 x 1024 x 1024 12/16, but 1024 x 1024 x 1 (3.4) 11.8/10.8 and 1236 x 1 x 2635
+ *     (3.2, moments) 38/23;
+ *   - with moments and more than 2.3 in several rounds of blocks: FP32
+ *     2 x 1024 x 1024 28.6/33.0 (one moment 23.2/23.2);
+ *   - on planes of up to 128 nodes, a long march of a barrier and a load latency
+ *     each (0.7-1.7 us per plane): 12000 x 10 x 10 FP32 17.4/33.5, one moment
+ *     13.9/17.8, FP64 34/43, 24/26; but FP64 2236 x 2 x 70 14.8/12.2.
+ * Elsewhere 0.47-0.95 of the time, a few FP32 shapes of 40-90 MB of factors
+ * 1.0-1.07 (190 shapes). */
+extern "C" int slbd_mp2_pays(int esj, int esk, int nmom, const MP2Plan *p) {
+  const double work = (p->jt + 2.0) * (p->kt + 2.0) * (p->ci + 2.0) / ((double)p->jt * p->kt * p->ci);
+  const long blocks = (long)p->njt * p->nkt * p->nch;
+  if (work > (nmom > 1 ? 3.3 : 3.5)) return 0;
+  if (nmom > 1 && work > 2.3 && blocks > 256) return 0;
+  return (long)esj * esk > 128;
 }
 
 template <typename T, int NMOM, int AX>

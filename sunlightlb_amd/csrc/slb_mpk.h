@@ -45,7 +45,8 @@ struct MP2Plan {
   int jt, kt, ci, njt, nkt, nch;
 };
 
-int slbd_mp2_plan(int esi, int esj, int esk, int prec, int nmom, MP2Plan *best);
+extern "C" int slbd_mp2_plan(int esi, int esj, int esk, int prec, int nmom, MP2Plan *best);
+extern "C" int slbd_mp2_pays(int esj, int esk, int nmom, const MP2Plan *p);
 /* two steps from records q to records qout on the factors wt */
 void slbd_mp2_launch(const void *wt, const void *q, void *qout, const uint32_t *mpf, int prec,
                      int nmom, const Geom &G, const MPArgs &A, const MP2Plan &Q, hipStream_t st);

@@ -28,11 +28,22 @@ def test_kernel_of_a_run(env, moving, want, monkeypatch):
     lat.free()
 
 
+def test_thin_lattices_keep_single_steps(monkeypatch):
+    import sunlightlb_amd as s
+    for on, want in ((None, "k_step"), ("1", "k_step2")):
+        if on:
+            monkeypatch.setenv("SLB_STEP2", on)
+        lat = s.Lattice(5000, 8, 8, precision=32)
+        assert lat.L.slb_run_kernel(lat.h).decode() == want
+        lat.free()
+
+
 @pytest.mark.parametrize("dims,prec,steps,env,want", [
     ((64, 64, 64), 32, 64, {}, "k_mpstep_w"), ((64, 64, 64), 32, 31, {}, "k_mpstep"),
     ((88, 88, 88), 32, 64, {}, "k_mpstep2"), ((88, 88, 88), 64, 64, {}, "k_mpstep2"),
     ((88, 88, 88), 32, 64, {"SLB_MP_STEP2": "0"}, "k_mpstep_w"),
     ((9, 8, 7), 32, 64, {"SLB_MP_STEP2": "1"}, "k_mpstep2"),
+    ((1, 800, 800), 32, 64, {}, "k_mpstep_w"), ((1, 800, 800), 32, 64, {"SLB_MP_STEP2": "1"}, "k_mpstep2"),
     ((88, 88, 88), 32, 64, {"SLB_MP_WEIGHTS": "0"}, "k_mpstep"),
     ((88, 88, 88), 32, 64, {"SLB_INDEX64": "1"}, "k_mpstep_w"),
 ])

@@ -39,3 +39,21 @@ def test_ragged_rows_do_not_take_the_narrowest_tiles():
     L, p = C.CDLL(LIB), Plan()
     L.slbd_step2_plan(20, 109, 665, 32, C.byref(p))
     assert p.kt >= 64
+
+
+TRACER = [  # esi, esj, esk, precision, moments tracked (values per node), as above
+    (128, 128, 128, 32, 3, 1), (256, 256, 256, 32, 3, 1), (128, 128, 128, 64, 1, 1),
+    (1236, 1, 2635, 32, 3, 1), (1024, 1024, 1, 32, 1, 1), (2236, 2, 70, 64, 3, 1),
+    (2, 1024, 1024, 32, 1, 1), (100, 90, 70, 32, 3, 1),
+    (1, 1024, 1024, 32, 3, 0), (1, 1024, 1024, 32, 1, 0), (1, 2907, 2023, 64, 3, 0),
+    (1024, 1024, 1, 32, 3, 0), (2, 1024, 1024, 32, 3, 0), (12000, 10, 10, 32, 3, 0),
+    (12000, 10, 10, 64, 1, 0), (1200000, 1, 1, 32, 3, 0), (1, 1, 1200000, 32, 1, 0),
+    (663, 3, 334, 32, 3, 0),
+]
+
+
+@pytest.mark.parametrize("esi,esj,esk,prec,nmom,pays", TRACER)
+def test_two_tracer_steps_per_pass_where_they_are_faster(esi, esj, esk, prec, nmom, pays):
+    L, p = C.CDLL(LIB), Plan()
+    ok = L.slbd_mp2_plan(esi, esj, esk, prec, nmom, C.byref(p))
+    assert (ok and L.slbd_mp2_pays(esj, esk, nmom, C.byref(p))) == pays
