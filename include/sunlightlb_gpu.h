@@ -170,8 +170,9 @@ double slb_mp_time_steps(MPSys mp, int nsteps);
 
 /* A batch of independent periodic boxes, each with nrhs right-hand sides
  * (object velocity sets), stepped together: one kernel launch over all
- * problems per two steps (SLB_BATCH_STEP2=0: per step), the step loop replayed
- * from a captured HIP graph. */
+ * problems per two steps where that is the faster way (SLB_BATCH_STEP2=1:
+ * always, 0: never), else per step, the step loop replayed from a captured HIP
+ * graph. */
 typedef struct slb_batch_s *SLBBatch;
 
 /* New empty batch; prec 32 or 64 (populations; force sums are FP64). */

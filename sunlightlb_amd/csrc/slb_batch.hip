@@ -589,47 +589,122 @@ static void build_tiles(slbd_batch *B) {
   invalidate_graphs(B);
 }
 
-/* Two steps per pass: tiles of every box (the split of a plane that costs
- * least, as slbd_step2_plan) in chunks along i, and the wall terms. */
+/* k_bstep2's times, us, [FP64][moving walls]: a launch; a block's start, a plane's
+ * barrier and load latency, a plane's work per thread (fitted to 250 batches of 1
+ * to 512 problems; standard error 11%).  One step of k_bstep: a launch and its
+ * first loads, then 30 values per node at 5.65 TB/s (7%). */
+static const double PLAN_US[2][2][4] = {{{2.8, 0.4, 0.91, 0.0024}, {2.5, 0.5, 1.20, 0.0026}},
+                                        {{1.5, 1.2, 1.03, 0.0046}, {2.0, 1.5, 1.13, 0.0043}}};
+static const double SINGLE_US[2] = {3.5, 5.9}; /* walls at rest, moving */
+/* Time of one block of k_bstep2, us: its start, then a barrier, the loads' latency
+ * and the work of pts threads per plane. */
+static double block_us(int prec, int moving, int pts, int ci) {
+  const double *t = PLAN_US[prec == 64][moving != 0];
+  return t[1] + (ci + 2) * (t[2] + t[3] * pts);
+}
+
+/* Whether a batch takes two steps per pass, and the tiles of every box (box: esi, esj, esk, right-hand sides, moving; tile: jt, kt,
+ * ci), and the time of two steps in this way and as two single ones (us).  Tried
+ * are tiles of at most `cap` threads and chunks of at most `len` planes; a CU
+ * holds one block at a time.  Large tiles and long chunks do the least work, but
+ * few problems then leave most CUs idle: one box of 64^3, FP32, us per step: 20
+ * blocks (13 x 64 x 16) 21.4, 256 (8 x 64 x 2) 6.3, single steps 7.6; one right-hand
+ * side of 6 of 64^3 35.1/19.3 (single / this), 2 x 2 of 256 x 256 x 4 25.3/15.2 (62 in
+ * chunks of a quarter).  Many problems of a few hundred nodes each fill no
+ * block and keep single steps: 384 of 8^3 6.5/14.2, 1536 of 6^3 12.3/32.2. */
+extern "C" int slbd_bstep2_plan(int nbox, const int *box, int prec, int *tile, double us[2]) {
+  static const int caps[] = {1024, 704, 512, 320, 192, 96};
+  static const int lens[] = {1 << 30, 64, 48, 32, 24, 16, 12, 8, 6, 4, 3, 2, 1};
+  const int most = prec == 32 ? B2Cfg<float>::NTHR : B2Cfg<double>::NTHR, cus = 256;
+  int *jk = (int *)malloc(sizeof(int) * 2 * (size_t)nbox);
+  if (!jk) { fprintf(stderr, "sunlightlb: out of host memory\n"); exit(EXIT_FAILURE); }
+  double best = 0.0, nodes = 0.0;
+  int moving = 0;
+  for (int b = 0; b < nbox; b++) {
+    const int *q = box + 5 * b;
+    nodes += (double)q[0] * q[1] * q[2] * q[3];
+    moving |= q[4] != 0;
+  }
+  for (size_t c = 0; c < sizeof caps / sizeof caps[0]; c++) {
+    if (caps[c] > most) continue;
+    for (int b = 0; b < nbox; b++) {
+      const int *q = box + 5 * b;
+      double bc = 0.0;
+      int jt = 0, kt = 0;
+      for (int nk = 1; nk <= (q[2] + 31) / 32 || jt == 0; nk++) {
+        const int k = (q[2] + nk - 1) / nk, nkt = (q[2] + k - 1) / k;
+        for (int jq = 1; jq <= q[1] && (jq + 2) * (k + 2) <= caps[c]; jq++) {
+          const int njt = (q[1] + jq - 1) / jq, j = (q[1] + njt - 1) / njt;
+          const double cost = (1.0 + 16.0 / k) * njt * nkt *
+                              block_us(prec, q[4], (j + 2) * (k + 2), 1 << 20);
+          if (jt == 0 || cost < bc) { bc = cost; jt = j; kt = k; }
+        }
+      }
+      jk[2 * b] = jt; jk[2 * b + 1] = kt;
+    }
+    for (size_t l = 0; l < sizeof lens / sizeof lens[0]; l++) {
+      double sum = 0.0, longest = 0.0;
+      long blocks = 0;
+      for (int b = 0; b < nbox; b++) {
+        const int *q = box + 5 * b, jt = jk[2 * b], kt = jk[2 * b + 1];
+        const int nch = lens[l] < q[0] ? (q[0] + lens[l] - 1) / lens[l] : 1, ci = (q[0] + nch - 1) / nch;
+        const long n = (long)((q[1] + jt - 1) / jt) * ((q[2] + kt - 1) / kt) * ((q[0] + ci - 1) / ci) * q[3];
+        const double t = block_us(prec, q[4], (jt + 2) * (kt + 2), ci);
+        blocks += n;
+        sum += n * t;
+        if (t > longest) longest = t;
+      }
+      const double t = blocks <= cus ? longest : sum / cus + 0.5 * longest;
+      if (best > 0.0 && t >= best) continue;
+      best = t;
+      for (int b = 0; b < nbox; b++) {
+        const int *q = box + 5 * b;
+        const int nch = lens[l] < q[0] ? (q[0] + lens[l] - 1) / lens[l] : 1;
+        tile[3 * b] = jk[2 * b]; tile[3 * b + 1] = jk[2 * b + 1];
+        tile[3 * b + 2] = (q[0] + nch - 1) / nch;
+      }
+    }
+  }
+  free(jk);
+  us[0] = PLAN_US[prec == 64][moving][0] + best;
+  us[1] = 2.0 * (SINGLE_US[moving] + nodes * 30.0 * (prec / 8) / 5.65e6);
+  /* with a margin for the estimate: of 338 batches, 2 at 4 to 80 us per step were
+   * then slower by more than 4% (6, 8%); FP32 at rest without it 7, by up to 21% */
+  return us[0] < (prec == 32 && !moving ? 0.85 : 0.95) * us[1];
+}
+
+/* Two steps per pass: tiles of every box in chunks along i, and the wall terms. */
 static void plan_pairs(slbd_batch *B) {
   const char *e = getenv("SLB_BATCH_STEP2");
   B->pairs = !(e && atoi(e) == 0);
   for (int p = 0; p < B->nprob; p++)   /* 32-bit byte offsets in a problem */
     if (15 * pop_nodes(B->hprobs[p].N) * (long)bts(B->prec) >= (1L << 32)) B->pairs = 0;
   if (!B->pairs) return;
-  const int cap = B->prec == 32 ? B2Cfg<float>::NTHR : B2Cfg<double>::NTHR;
-  const int cus = 256;
-  int pts = 0;
-  long best = 0, total[4] = {0, 0, 0, 0}, longest[4] = {0, 0, 0, 0};
-  for (int p = 0; p < B->nprob; p++) {
-    BProb *q = &B->hprobs[p];
-    double bc = 0.0;
-    q->jt = 0;
-    for (int nk = 1; nk <= (q->esk + 31) / 32 || q->jt == 0; nk++) {
-      const int kt = (q->esk + nk - 1) / nk, nkt = (q->esk + kt - 1) / kt;
-      for (int jq = 1; jq <= q->esj && (jq + 2) * (kt + 2) <= cap; jq++) {
-        const int njt = (q->esj + jq - 1) / jq, jt = (q->esj + njt - 1) / njt;
-        const double cost = (1.0 + 16.0 / kt) * njt * nkt *
-                            ((double)(jt + 2) * (kt + 2) + (double)jt * kt + 1000.0);
-        if (q->jt == 0 || cost < bc) { bc = cost; q->jt = jt; q->kt = kt; }
-      }
-    }
-    if ((q->jt + 2) * (q->kt + 2) > pts) pts = (q->jt + 2) * (q->kt + 2);
-    const long t = (long)((q->esj + q->jt - 1) / q->jt) * ((q->esk + q->kt - 1) / q->kt);
-    for (int c = 0; c < 4; c++) {
-      const int ci = (q->esi + c) / (c + 1);
-      total[c] += t * ((q->esi + ci - 1) / ci);
-      if (ci + 2 > longest[c]) longest[c] = ci + 2;
-    }
+  int *box = (int *)malloc(sizeof(int) * 8 * (size_t)B->nbox), *tile = box + 5 * (size_t)B->nbox;
+  if (!box) { fprintf(stderr, "sunlightlb: out of host memory\n"); exit(EXIT_FAILURE); }
+  for (int b = 0; b < B->nbox; b++) {
+    const BBox *x = &B->box[b];
+    const int q[5] = {x->esi, x->esj, x->esk, x->nrhs, x->moving};
+    memcpy(box + 5 * b, q, sizeof q);
   }
-  for (int c = 1; c < 4; c++)
-    if ((total[c] + cus - 1) / cus * longest[c] < (total[best] + cus - 1) / cus * longest[best])
-      best = c;
-  int4 *h = (int4 *)malloc(sizeof(int4) * (total[best] > 0 ? total[best] : 1));
+  double us[2];
+  if (!slbd_bstep2_plan(B->nbox, box, B->prec, tile, us) && !e) B->pairs = 0;
+  int pts = 0;
+  long total = 0;
+  for (int b = 0, p = 0; b < B->nbox; b++)
+    for (int r = 0; r < B->box[b].nrhs; r++, p++) {
+      BProb *q = &B->hprobs[p];
+      q->jt = tile[3 * b]; q->kt = tile[3 * b + 1]; q->ci = tile[3 * b + 2];
+      if ((q->jt + 2) * (q->kt + 2) > pts) pts = (q->jt + 2) * (q->kt + 2);
+      total += (long)((q->esj + q->jt - 1) / q->jt) * ((q->esk + q->kt - 1) / q->kt) *
+               ((q->esi + q->ci - 1) / q->ci);
+    }
+  free(box);
+  if (!B->pairs) return;
+  int4 *h = (int4 *)malloc(sizeof(int4) * (total > 0 ? total : 1));
   long n = 0;
   for (int p = 0; p < B->nprob; p++) {
-    BProb *q = &B->hprobs[p];
-    q->ci = (int)((q->esi + best) / (best + 1));
+    const BProb *q = &B->hprobs[p];
     for (int i0 = 0; i0 < q->esi; i0 += q->ci)
       for (int j0 = 0; j0 < q->esj; j0 += q->jt)
         for (int k0 = 0; k0 < q->esk; k0 += q->kt) h[n++] = make_int4(p, j0, k0, i0);

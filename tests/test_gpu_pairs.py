@@ -159,7 +159,7 @@ def test_batch_pairs_many_right_hand_sides(monkeypatch):
     (32768): populations of the problems at that edge, bit for bit."""
     import sunlightlb_amd as s
     nrhs, out = 32770, []
-    for on in "01":
+    for on in "01":          # 1: also where single steps are the faster way
         monkeypatch.setenv("SLB_BATCH_STEP2", on)
         print(f"batch pairs: {nrhs} right-hand sides, pairs {on}", flush=True)
         lat = s.Lattice(6, 5, 4, precision=32)

@@ -57,15 +57,19 @@ def test_kernel_of_a_tracer_run(dims, prec, steps, env, want, monkeypatch):
     lat.free()
 
 
-@pytest.mark.parametrize("env,want", [({}, "k_bstep2"), ({"SLB_BATCH_STEP2": "0"}, "k_bstep")])
-def test_kernel_of_a_batch(env, want, monkeypatch):
+@pytest.mark.parametrize("dims,boxes,env,want", [
+    ((40, 40, 48), 6, {}, "k_bstep2"), ((40, 40, 48), 6, {"SLB_BATCH_STEP2": "0"}, "k_bstep"),
+    ((64, 64, 64), 1, {}, "k_bstep2"), ((6, 6, 6), 64, {}, "k_bstep"),
+    ((6, 6, 6), 64, {"SLB_BATCH_STEP2": "1"}, "k_bstep2"),
+])
+def test_kernel_of_a_batch(dims, boxes, env, want, monkeypatch):
     for k, v in env.items():
         monkeypatch.setenv(k, v)
-    lat = build((40, 40, 48), 32, 1, 1, 0, 0)
+    lat = build(dims, 32, 1, 1, 0, 0)
     L, n = lat.L, len(lat.objects())
     b = L.slb_batch_new(32)
     vel = np.zeros((6, n, 6))
-    for _ in range(6):
+    for _ in range(boxes):
         L.slb_batch_add(b, lat.h, 6, vel.ctypes.data_as(C.POINTER(C.c_double)))
     lat.free()
     assert L.slb_batch_commit(b) == 0

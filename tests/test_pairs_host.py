@@ -57,3 +57,35 @@ def test_two_tracer_steps_per_pass_where_they_are_faster(esi, esj, esk, prec, nm
     L, p = C.CDLL(LIB), Plan()
     ok = L.slbd_mp2_plan(esi, esj, esk, prec, nmom, C.byref(p))
     assert (ok and L.slbd_mp2_pays(esj, esk, nmom, C.byref(p))) == pays
+
+
+BATCH = [  # boxes (esi, esj, esk, right-hand sides, moving), precision, pairs, least blocks
+    ([(64, 64, 64, 1, 0)], 32, 1, 128), ([(64, 64, 64, 1, 1)], 64, 1, 128),
+    ([(48, 48, 48, 1, 1)], 32, 1, 100), ([(128, 128, 128, 1, 0)], 32, 1, 200),
+    ([(64, 64, 64, 6, 1)], 32, 1, 200), ([(256, 256, 4, 2, 0)] * 2, 32, 1, 200),
+    ([(112, 7, 15, 1, 1)] * 2, 64, 1, 60), ([(94, 49, 5, 1, 0)] * 5, 64, 1, 120),
+    ([(48, 54, 33, 6, 1), (40, 61, 62, 6, 1), (33, 35, 64, 6, 1)] * 10, 32, 1, 200),
+    ([(6, 6, 6, 6, 0)] * 256, 32, 0, 0), ([(8, 8, 8, 6, 1)] * 64, 64, 0, 0),
+    ([(64, 64, 1, 6, 0)] * 64, 32, 0, 0), ([(96, 5, 5, 3, 0)] * 40, 64, 0, 0),
+    ([(5, 3, 701, 1, 1)], 64, None, 0), ([(1, 1, 1, 1, 0)], 32, None, 0), ([(2, 300, 1, 1, 1)], 64, None, 0),
+]
+
+
+@pytest.mark.parametrize("boxes,prec,pays,least", BATCH)
+def test_batch_plan(boxes, prec, pays, least):
+    """Tiles that fit a block and cover their box, enough of them to use the
+    CUs where the problems are few, and single steps where those are faster."""
+    L, n = C.CDLL(LIB), len(boxes)
+    box = (C.c_int * (5 * n))(*[v for b in boxes for v in b])
+    tile, us = (C.c_int * (3 * n))(), (C.c_double * 2)()
+    got = L.slbd_bstep2_plan(n, box, prec, tile, us)
+    blocks = 0
+    for q, (esi, esj, esk, nrhs, _) in enumerate(boxes):
+        jt, kt, ci = tile[3 * q:3 * q + 3]
+        assert 1 <= jt <= esj and 1 <= kt <= esk and 1 <= ci <= esi
+        assert (jt + 2) * (kt + 2) <= (1024 if prec == 32 else 512)
+        blocks += -(-esi // ci) * -(-esj // jt) * -(-esk // kt) * nrhs
+    if pays is not None:
+        assert got == pays and (us[0] < us[1]) == pays
+    if pays:
+        assert blocks >= least
