@@ -79,10 +79,10 @@ __device__ __forceinline__ int tap_node(const NGeom &G, int z, int y, int x, int
 /* loads are in flight together.                                            */
 
 /* CI: the input channels where they are 16, 32 or 64 (taps without divisions,
- * two K chunks' loads in flight), else 0.  Bound by the latency of a chunk's
- * loads on few nodes: 64 -> 64 channels on 1080 and 8640 nodes 51 -> 34 us with
- * CI and one tile per wave, 16 -> 16 on 553 thousand nodes 46 -> 43 us.  The K
- * order and MFMA sequence per tile do not depend on CI or NTW. */
+ * two K chunks' loads in flight), else 0 (slbn_conv_ci).  Bound by the latency of
+ * a chunk's loads on few nodes: 64 -> 64 channels on 1080 and 8640 nodes 54 -> 33
+ * us with CI and one tile per wave (slbn_conv_ntw), 16 -> 16 on 553 thousand nodes
+ * 48 -> 41 us.  The K order and MFMA sequence per tile do not depend on CI or NTW. */
 template <int MT, int NTW, int CI>
 __global__ void __launch_bounds__(256)
 k_conv(const uint16_t *__restrict__ X, int cin, const uint16_t *__restrict__ W, int kpad,
@@ -109,7 +109,7 @@ k_conv(const uint16_t *__restrict__ X, int cin, const uint16_t *__restrict__ W, 
   for (int u = 0; u < NTW; u++)
 #pragma unroll
     for (int m = 0; m < MT; m++) acc[u][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll(CI ? 2 : 1)
+#pragma unroll CI ? 2 : 1
   for (int k0 = 0; k0 < Kp; k0 += 32) {
     const int kk = k0 + 8 * grp;
     /* the weights of this K chunk, loaded once for all NTW node tiles */
@@ -1052,9 +1052,25 @@ static NGeom ngeom(int D, int H, int Wd) {
 
 /* node tiles of 16 per wave in the convolution (weights of a K chunk are
  * loaded once for all of them) */
-#ifndef SLBN_CONV_NTW
-#define SLBN_CONV_NTW 4
-#endif
+/* Node tiles of 16 per wave (four waves per block).  Every wave loads all the
+ * weights, so more tiles are less traffic from L2, as long as every CU has a
+ * block: one tile up to 256 blocks of 64 nodes, two up to 256 of 128, then four.
+ * One / two / four tiles, us, 64 -> 64 channels on 14400 nodes 33/40/54, 30000
+ * 63/40/54, 50400 121/76/56, 125 thousand 238/147/104; 16 -> 32 on 30000
+ * 10.4/9.2/12.3, 125 thousand 32/21/17.5.  Few weights gain from two up to three such
+ * blocks per CU: 16 -> 16 on 69120 12.6/11.0/12.5, 32 -> 16 17.3/16.7/18.7 (on 125
+ * thousand 18.7/13.5/12.8, 27/21.5/21). */
+extern "C" int slbn_conv_ntw(int cin, int cout, long N) {
+  if (N <= 16384) return 1;
+  return N <= 32768 || (cin + cout <= 48 && N <= 98304) ? 2 : 4;
+}
+/* The channel count as a template parameter, or 0: 32 -> 64 with four tiles in
+ * flight is slower with it where the chip is full, 180 thousand nodes 58 against
+ * 50 us, a million 250 against 228 (50400 22.5 against 25.4). */
+extern "C" int slbn_conv_ci(int cin, int cout, long N) {
+  if (cin == 32 && cout > 48 && N >= 131072) return 0;
+  return cin == 16 || cin == 32 || cin == 64 ? cin : 0;
+}
 
 static hipStream_t nn_stream = 0;
 extern "C" void slbn_set_stream(void *s) { nn_stream = (hipStream_t)s; }
@@ -1068,8 +1084,6 @@ extern "C" void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const f
                           int Wd) {
   const NGeom G = ngeom(D, H, Wd);
   const int Kp = slbn_kpad(cin);
-  /* 4 waves per block, each NTW node tiles of 16 */
-  const unsigned g = blocks_for(G.N, 64 * SLBN_CONV_NTW);
   const int sgn = transposed ? -1 : 1;
   if (cin < 8 || cin % 8 || cout < 1 || cout % 4 || (long)G.N * (cin > cout ? cin : cout) >= (1L << 31)) {
     fprintf(stderr, "slbn_conv: cin must be a multiple of 8, cout of 4, tensors < 2^31 elements\n");
@@ -1107,24 +1121,21 @@ extern "C" void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const f
     LAUNCHCHECK();
     return;
   }
-  /* few nodes: one tile per wave, for four times the blocks (64 -> 64 channels
-   * on 1080 nodes: 5 blocks of four tiles per wave) */
-  const bool few = g < 512;
-  const unsigned gf = few ? blocks_for(G.N, 64) : g;
+  const int ntw = slbn_conv_ntw(cin, cout, G.N), ci = slbn_conv_ci(cin, cout, G.N);
+#define SLBN_CONVN(MT, NTW, CI)                                                                  \
+  hipLaunchKernelGGL((k_conv<MT, NTW, CI>), dim3(blocks_for(G.N, 64 * NTW)), dim3(256), 0,       \
+                     nn_stream, X, cin, W, Kp, bias, Y, Yf, cout, relu, sgn, G)
 #define SLBN_CONVC(MT, CI)                                                                       \
   do {                                                                                           \
-    if (few)                                                                                     \
-      hipLaunchKernelGGL((k_conv<MT, 1, CI>), dim3(gf), dim3(256), 0, nn_stream, X, cin, W, Kp,  \
-                         bias, Y, Yf, cout, relu, sgn, G);                                       \
-    else                                                                                         \
-      hipLaunchKernelGGL((k_conv<MT, SLBN_CONV_NTW, CI>), dim3(g), dim3(256), 0, nn_stream, X,   \
-                         cin, W, Kp, bias, Y, Yf, cout, relu, sgn, G);                           \
+    if (ntw == 1) SLBN_CONVN(MT, 1, CI);                                                         \
+    else if (ntw == 2) SLBN_CONVN(MT, 2, CI);                                                    \
+    else SLBN_CONVN(MT, 4, CI);                                                                  \
   } while (0)
 #define SLBN_CONV(MT)                                                                            \
   do {                                                                                           \
-    if (cin == 16) SLBN_CONVC(MT, 16);                                                           \
-    else if (cin == 32) SLBN_CONVC(MT, 32);                                                      \
-    else if (cin == 64) SLBN_CONVC(MT, 64);                                                      \
+    if (ci == 16) SLBN_CONVC(MT, 16);                                                            \
+    else if (ci == 32) SLBN_CONVC(MT, 32);                                                       \
+    else if (ci == 64) SLBN_CONVC(MT, 64);                                                       \
     else SLBN_CONVC(MT, 0);                                                                      \
   } while (0)
   if (mt == 1) SLBN_CONV(1);
@@ -1132,6 +1143,7 @@ extern "C" void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const f
   else if (mt == 3) SLBN_CONV(3);
   else if (mt == 4) SLBN_CONV(4);
   else { fprintf(stderr, "slbn_conv: at most 64 output channels\n"); exit(EXIT_FAILURE); }
+#undef SLBN_CONVN
 #undef SLBN_CONVC
 #undef SLBN_CONV
   LAUNCHCHECK();

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import nn as onn
-from test_gpu_warm import Dev, bf_random, lib
+from test_gpu_warm import Dev, bf_random, lib, test_conv_forward_matches_oracle as conv_matches_oracle
 
 pytestmark = pytest.mark.gpu
 
@@ -60,6 +60,21 @@ def test_general_convolution_equals_the_staged_one(shape, cin, cout, monkeypatch
     assert got[0][1].any()
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (32, 64), (64, 32)])
+@pytest.mark.parametrize("shape", [(4, 128, 64), (8, 128, 64), (16, 128, 128)])
+def test_two_and_four_node_tiles_equal_the_staged_one(shape, cin, cout, monkeypatch):
+    """Two node tiles per wave, and the generic channel count (32 -> 64 on 262
+    thousand nodes)."""
+    test_general_convolution_equals_the_staged_one(shape, cin, cout, monkeypatch)
+
+
+@pytest.mark.parametrize("cin,cout", [(16, 16), (24, 8), (64, 64)])
+@pytest.mark.parametrize("shape", [(13, 37, 41), (3, 79, 71)])
+def test_two_node_tiles_with_a_remainder(shape, cin, cout):
+    """19721 and 16827 nodes: the last wave's second tile partly and wholly past the end."""
+    conv_matches_oracle(shape, cin, cout, 1)
 
 
 @pytest.mark.parametrize("cs,c", [(2, 16), (16, 16), (8, 16), (10, 16), (3, 12), (24, 8)])
