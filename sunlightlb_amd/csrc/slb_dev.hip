@@ -3101,7 +3101,7 @@ k_features(const uint16_t *__restrict__ flags, const int *__restrict__ ns,
     const uint32_t u = __float_as_uint(v[q]);
     h[q] = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
   }
-  if (C % 8 == 0 && ((uintptr_t)X & 15) == 0) {   /* a node's channels in 16-byte stores */
+  if (C >= 8 && C % 8 == 0 && ((uintptr_t)X & 15) == 0) { /* a node's channels in 16-byte stores */
     uint4 *p = (uint4 *)(X + n * C);
     p[0] = make_uint4((h[0] & 0xffffu) | (h[1] << 16), 0, 0, 0);
     for (int c = 1; c < C / 8; c++) p[c] = make_uint4(0, 0, 0, 0);
@@ -3150,6 +3150,24 @@ k_targets(const T *__restrict__ a, const uint16_t *__restrict__ flags, double rh
     m[8] = (float)(P[4] * ss);
     m[9] = (float)(P[5] * ss);
   }
+  auto put = [&](long e, float v) {
+    if constexpr (sizeof(O) == 4) {
+      Y[e] = v;
+    } else {
+      const uint32_t w = __float_as_uint(v) + 0x7fffu + ((__float_as_uint(v) >> 16) & 1u);
+      Y[e] = (uint16_t)(w >> 16);
+    }
+  };
+  /* up to four channels the lanes' stores share their lines, and the LDS only
+   * adds its latency (C = 4, 128^3: 34.1 against 36.2 us); none for C <= 0 */
+  if (C <= 4) {
+    if (n < G.N) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (q < C) put(n * C + q, m[q]);
+    }
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < 10; q++) sm[threadIdx.x * 10 + q] = m[q];
   __syncthreads();
@@ -3158,13 +3176,7 @@ k_targets(const T *__restrict__ a, const uint16_t *__restrict__ flags, double rh
   int x = (int)threadIdx.x / C, c = (int)threadIdx.x - x * C;
   const int dx = 256 / C, dc = 256 - dx * C;
   for (long e = threadIdx.x; e < (long)nodes * C; e += 256) {
-    const float v = c < 10 ? sm[x * 10 + c] : 0.f;
-    if constexpr (sizeof(O) == 4) {
-      Y[nb * C + e] = v;
-    } else {
-      const uint32_t w = __float_as_uint(v) + 0x7fffu + ((__float_as_uint(v) >> 16) & 1u);
-      Y[nb * C + e] = (uint16_t)(w >> 16);
-    }
+    put(nb * C + e, c < 10 ? sm[x * 10 + c] : 0.f);
     x += dx;
     c += dc;
     if (c >= C) { c -= C; x++; }

@@ -136,3 +136,47 @@ def test_moments_of_any_channel_count(dims):
         assert np.array_equal(out[ch][:, :q], out[10][:, :q])
     assert np.abs(out[10]).max() > 0.0
     lat.free()
+
+
+@pytest.mark.parametrize("ch", [0, -8, -16])
+def test_no_channels_write_nothing(ch):
+    """Channel counts of zero and below leave the tensors as they are."""
+    import sunlightlb_amd as s
+    lat = s.Lattice(6, 7, 9, precision=64)
+    lat.L.insertsph(lat.h, 2.0, 3.0, 3.0, 4.0)
+    lat.s.dpdx = 1e-3
+    n = 64 * lat.N
+    pat = np.arange(n, dtype=np.uint32)
+    d = Dev(host=pat)
+    mid = d.p + 2 * n
+    ell = lat.L.slb_warm_features(lat.h, mid, ch)
+    assert ell > 0.0 and ell == lat.L.slb_warm_features_noalloc(lat.h, mid, ch)
+    lat.L.slb_warm_moments(lat.h, mid, ch, 1.0)
+    lat.L.slb_warm_targets(lat.h, mid, ch, 1.0)
+    assert np.array_equal(d.get(np.uint32, (n,)), pat)
+    d.free()
+    lat.free()
+
+
+@pytest.mark.parametrize("ch", [1, 2, 4, 5])
+def test_moments_on_few_channels(ch):
+    """Both sides of the line between stores from registers and through the LDS,
+    FP32 and BF16, a last block that is not full; nothing past the end."""
+    import sunlightlb_amd as s
+    lat = s.Lattice(5, 9, 23, precision=32)
+    lat.L.insertsph(lat.h, 1.5, 1.0, 2.0, 3.0)
+    lat.s.dpdx = 1e-3
+    lat.set_pops(1e-3 * np.random.default_rng(5).standard_normal(lat.N * 15))
+    out = {}
+    for c in (10, ch):
+        m, t = Dev(lat.N * c * 4 + 64), Dev(lat.N * c * 2 + 64)
+        lat.L.slb_warm_moments(lat.h, m.p, c, 1.0)
+        lat.L.slb_warm_targets(lat.h, t.p, c, 1.0)
+        a, b = m.get(np.float32, (lat.N * c + 16,)), t.get(np.uint16, (lat.N * c + 32,))
+        assert not a[lat.N * c:].any() and not b[lat.N * c:].any()
+        out[c] = a[:lat.N * c].reshape(lat.N, c), b[:lat.N * c].reshape(lat.N, c)
+        m.free()
+        t.free()
+    for a, b in zip(out[ch], out[10]):
+        assert a.any() and np.array_equal(a, b[:, :ch])
+    lat.free()
