@@ -31,8 +31,10 @@ void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const float *bias,
  * 8 up to 128, even y extent) bricks of two x-rows are staged in LDS and all
  * 27 taps computed there; else when slbn_wgrad_blocked_ok() (channels 16, 32
  * or 64, any extents) it is a GEMM over a node-blocked copy of X and dY; both
- * with a fixed summation order.  Otherwise (48 channels) a per-tap LDS-staged
- * kernel with atomics. */
+ * with a fixed summation order, in a workspace kept per stream.  Otherwise (48
+ * channels; no memory for the workspace, or more than SLBN_WGRAD_WS bytes; rows
+ * that are no multiple of 8 while the stream is captured) a per-tap LDS-staged
+ * kernel with atomics.  Safe from several threads. */
 int  slbn_wgrad_lds16_ok(int cin, int cout, int D, int H, int Wd);
 int  slbn_wgrad_blocked_ok(int cin, int cout, int D, int H, int Wd);
 void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, int cout, float *dW, int D,

@@ -23,6 +23,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <mutex>
 #include "sunlightlb_nn.h"
 
 #define HIPCHECK(call)                                                        \
@@ -1149,21 +1150,71 @@ extern "C" void slbn_conv(const uint16_t *X, int cin, const uint16_t *W, const f
   LAUNCHCHECK();
 }
 
-/* workspace of the blocked weight gradient (grown on demand, kept) */
-static void *wg_ws = nullptr;
-static size_t wg_ws_bytes = 0;
+/* Workspaces of the weight gradient, grown on demand and kept: one per stream,
+ * since calls on two streams overlap, of at most WG_STREAMS streams (another one
+ * waits for the device and takes over the next in turn).  wg_mutex
+ * is held over a call's launches, so that two threads' calls on one stream
+ * follow one another in it.  NULL where there is none to be had: no memory, more
+ * than SLBN_WGRAD_WS bytes (read per call), or one that would have to grow or
+ * change hands while the stream is captured. */
+#define WG_STREAMS 16
+struct WgSpace {
+  int dev, used;
+  hipStream_t stream;
+  void *p;
+  size_t bytes;
+};
+static WgSpace wg_space[WG_STREAMS];
+static std::mutex wg_mutex;
+
+static bool nn_capturing(void) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  HIPCHECK(hipStreamIsCapturing(nn_stream, &st));
+  return st != hipStreamCaptureStatusNone;
+}
+
 static void *wg_workspace(size_t bytes) {
-  if (bytes > wg_ws_bytes) {
-    HIPCHECK(hipStreamSynchronize(nn_stream));
-    if (wg_ws) HIPCHECK(hipFree(wg_ws));
-    HIPCHECK(hipMalloc(&wg_ws, bytes));
-    wg_ws_bytes = bytes;
+  const char *e = getenv("SLBN_WGRAD_WS");
+  if (e && bytes > strtoull(e, NULL, 10)) return nullptr;
+  int dev = 0;
+  HIPCHECK(hipGetDevice(&dev));
+  WgSpace *w = nullptr;
+  for (int q = 0; q < WG_STREAMS && !w; q++) {
+    WgSpace *c = &wg_space[q];
+    if (!c->used) { c->used = 1; c->dev = dev; c->stream = nn_stream; }
+    if (c->dev == dev && c->stream == nn_stream) w = c;
   }
-  return wg_ws;
+  if (!w) {
+    static int turn = 0;
+    if (nn_capturing()) return nullptr;
+    HIPCHECK(hipDeviceSynchronize());
+    w = &wg_space[turn++ % WG_STREAMS];
+    if (w->dev != dev) {
+      if (w->p) HIPCHECK(hipFree(w->p));
+      w->p = nullptr;
+      w->bytes = 0;
+    }
+    w->dev = dev;
+    w->stream = nn_stream;
+  }
+  if (bytes > w->bytes) {
+    if (nn_capturing()) return nullptr;
+    HIPCHECK(hipStreamSynchronize(nn_stream));
+    if (w->p) HIPCHECK(hipFree(w->p));
+    w->p = nullptr;
+    w->bytes = 0;
+    if (hipMalloc(&w->p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      w->p = nullptr;
+      return nullptr;
+    }
+    w->bytes = bytes;
+  }
+  return w->p;
 }
 
 /* the per-tap LDS-staged kernel with atomics: the channel counts that the
- * blocked one does not cover (48) */
+ * blocked one does not cover (48), and calls without a workspace */
 static void wgrad_staged(const uint16_t *X, int cin, const uint16_t *dY, int cout, float *dW,
                          const NGeom &G) {
   const int Kp = slbn_kpad(cin);
@@ -1205,10 +1256,13 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
     fprintf(stderr, "slbn_conv_wgrad: channels must be 16..64 in steps of 16\n");
     exit(EXIT_FAILURE);
   }
-  if (!slbn_wgrad_blocked_ok(cin, cout, D, H, Wd)) {
+  /* rows of any other length than multiples of 8 nodes need no workspace in a
+   * captured graph: one that a later call outgrows would leave it a freed address */
+  if (!slbn_wgrad_blocked_ok(cin, cout, D, H, Wd) || (Wd % 8 != 0 && nn_capturing())) {
     wgrad_staged(X, cin, dY, cout, dW, G);
     return;
   }
+  std::lock_guard<std::mutex> lock(wg_mutex);
   if (slbn_wgrad_lds16_ok(cin, cout, D, H, Wd)) {
     /* 16 -> 16 channels: LDS-staged bricks, about two blocks per CU */
     const int nbricks = D * (H / 2);
@@ -1216,6 +1270,7 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
     const int per = (nbricks + nb - 1) / nb;
     nb = (nbricks + per - 1) / per;
     float *part = (float *)wg_workspace((size_t)27 * nb * 256 * sizeof(float));
+    if (!part) { wgrad_staged(X, cin, dY, cout, dW, G); return; }
     hipLaunchKernelGGL(k_wgrad16_lds, dim3((unsigned)nb), dim3(256), wg16_lds_bytes(Wd), nn_stream,
                        X, dY, part, per, G);
     LAUNCHCHECK();
@@ -1224,10 +1279,11 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
     LAUNCHCHECK();
     return;
   }
-  /* rows of any length in groups of 8 nodes; the padded groups cost at most
-   * 8/9 of the work at rows of 9 nodes and replace 27 launches of the per-tap
-   * kernel (96 x 80 x 72 network, its level of 36-node rows: 27 x 63 us
-   * against 34 us) */
+  /* rows of any length in groups of 8 nodes: ceil(Wd / 8) 8 / Wd times the work and
+   * the copies of a row, 16/9 at 9 nodes and 8 at one, in place of the per-tap
+   * kernel's 27 launches; us per-tap / here, 64 -> 64 channels: rows of 36 (48 x 40)
+   * 2217/103, of 9 (64 x 64) 2195/73, of one node 128 x 128 2184/118, 512 x 512
+   * 5233/2525 (16 -> 16 2914/217), 8 x 8 122/19 */
   const bool pad = Wd % 8 != 0;
   const long ngr = (long)D * H * ((Wd + 7) >> 3);
   /* enough blocks per tap to fill the chip with 27 taps, each block a
@@ -1244,6 +1300,7 @@ extern "C" void slbn_conv_wgrad(const uint16_t *X, int cin, const uint16_t *dY, 
   const size_t xb = (size_t)ngr * 8 * cin * 2, db = (size_t)ngr * 8 * cout * 2;
   const size_t pb = (size_t)27 * nb * cout * cin * 4;
   char *ws = (char *)wg_workspace(xb + db + pb);
+  if (!ws) { wgrad_staged(X, cin, dY, cout, dW, G); return; }
   uint16_t *Xb = (uint16_t *)ws, *Db = (uint16_t *)(ws + xb);
   float *part = (float *)(ws + xb + db);
   const long rows = (long)D * H;

@@ -180,3 +180,112 @@ def test_moments_on_few_channels(ch):
     for a, b in zip(out[ch], out[10]):
         assert a.any() and np.array_equal(a, b[:, :ch])
     lat.free()
+
+
+def wgrad_data(shape, cin, cout, seed):
+    rng = np.random.default_rng(seed)
+    xb, x = bf_random(rng, shape + (cin,))
+    gb, g = bf_random(rng, shape + (cout,))
+    return Dev(host=xb), Dev(host=gb), onn.conv3d_bwd_weight(x, g).reshape(cout, 27 * cin)
+
+
+def wgrad_close(got, ref, times=1):
+    assert np.abs(got[:, :ref.shape[1]].astype(np.float64) - times * ref).max() < 1e-5 * times * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("shape", [(6, 5, 18), (4, 6, 16)])
+def test_weight_gradient_without_a_workspace(shape, monkeypatch):
+    L, cin, cout = lib(), 32, 16
+    monkeypatch.setenv("SLBN_WGRAD_WS", "1000")
+    dX, dG, ref = wgrad_data(shape, cin, cout, 4)
+    dW = Dev(cout * onn.kpad(cin) * 4)
+    L.slbn_conv_wgrad(dX.p, cin, dG.p, cout, dW.p, *shape)
+    L.slbn_sync()
+    wgrad_close(dW.get(np.float32, (cout, onn.kpad(cin))), ref)
+    for d in (dX, dG, dW):
+        d.free()
+
+
+def test_weight_gradient_on_two_streams():
+    """Calls on two streams overlap: each keeps its own workspace (fixed order
+    of summation, so bit for bit the result of a call alone)."""
+    import torch
+    L, cin, cout, shape, reps = lib(), 32, 32, (20, 20, 18), 12
+    kp = onn.kpad(cin)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    data = [wgrad_data(shape, cin, cout, q) for q in range(2)]
+    alone, both = [], [[Dev(cout * kp * 4) for _ in range(reps)] for _ in streams]
+    try:
+        for q, (dX, dG, ref) in enumerate(data):
+            dW = Dev(cout * kp * 4)
+            L.slbn_conv_wgrad(dX.p, cin, dG.p, cout, dW.p, *shape)
+            L.slbn_sync()
+            alone.append(dW.get(np.uint32, (cout, kp)))
+            wgrad_close(alone[q].view(np.float32), ref)
+            dW.free()
+        for r in range(reps):
+            for q, st in enumerate(streams):
+                L.slbn_set_stream(st.cuda_stream)
+                L.slbn_conv_wgrad(data[q][0].p, cin, data[q][1].p, cout, both[q][r].p, *shape)
+        torch.cuda.synchronize()
+    finally:
+        L.slbn_set_stream(None)
+    for q in range(2):
+        for d in both[q]:
+            assert np.array_equal(d.get(np.uint32, (cout, kp)), alone[q])
+            d.free()
+
+
+def test_weight_gradient_on_many_streams():
+    """More streams than workspaces."""
+    import torch
+    L, cin, cout, shape = lib(), 16, 16, (5, 6, 9)
+    kp = onn.kpad(cin)
+    dX, dG, ref = wgrad_data(shape, cin, cout, 2)
+    dW = Dev(cout * kp * 4)
+    streams = [torch.cuda.Stream() for _ in range(24)]
+    assert len({st.cuda_stream for st in streams}) > 16
+    try:
+        for st in streams:
+            L.slbn_set_stream(st.cuda_stream)
+            L.slbn_conv_wgrad(dX.p, cin, dG.p, cout, dW.p, *shape)
+            L.slbn_sync()
+    finally:
+        L.slbn_set_stream(None)
+    wgrad_close(dW.get(np.float32, (cout, kp)), ref, len(streams))
+    for d in (dX, dG, dW):
+        d.free()
+
+
+def test_weight_gradient_in_a_captured_graph():
+    """Ragged rows captured without a call before them, and replayed between
+    eager calls that grow the workspace."""
+    import torch
+    L, cin, cout, shape = lib(), 16, 32, (7, 6, 11)
+    kp = onn.kpad(cin)
+    dX, dG, ref = wgrad_data(shape, cin, cout, 9)
+    dW = Dev(cout * kp * 4)
+    st, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.graph(g, stream=st):
+            L.slbn_set_stream(torch.cuda.current_stream().cuda_stream)
+            L.slbn_conv_wgrad(dX.p, cin, dG.p, cout, dW.p, *shape)
+    finally:
+        L.slbn_set_stream(None)
+    torch.cuda.synchronize()
+    assert not dW.get(np.float32, (cout, kp)).any()
+    for r in range(1, 4):
+        g.replay()
+        torch.cuda.synchronize()
+        wgrad_close(dW.get(np.float32, (cout, kp)), ref, r)
+        big = (12 * r, 20, 23)
+        bX, bG, bref = wgrad_data(big, cin, cout, 20 + r)
+        bW = Dev(cout * kp * 4)
+        L.slbn_conv_wgrad(bX.p, cin, bG.p, cout, bW.p, *big)
+        L.slbn_sync()
+        wgrad_close(bW.get(np.float32, (cout, kp)), bref)
+        for d in (bX, bG, bW):
+            d.free()
+    for d in (dX, dG, dW):
+        d.free()
