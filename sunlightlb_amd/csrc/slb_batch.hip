@@ -498,6 +498,7 @@ struct slbd_batch {
   void *wrows;
   int4 *tiles2;
   int ntiles2, thr2;        /* tiles, threads per block */
+  size_t bytes, pair_bytes; /* device memory held; by what pairs need alone */
   BProb *hprobs;
   int *box_first_prob;
   /* launch configuration */
@@ -571,6 +572,66 @@ extern "C" int slbd_batch_add_box(slbd_batch *B, int esi, int esj, int esk,
   return B->nbox++;
 }
 
+/* Device memory of a batch.  A limit set from the host (tests; 0: none) stands
+ * for a device with that much left. */
+static size_t mem_limit, last_bytes;
+
+/* Set the limit; the bytes that the batch committed last holds. */
+extern "C" size_t slbd_batch_mem_limit(size_t bytes) {
+  mem_limit = bytes;
+  return last_bytes;
+}
+
+static bool try_alloc(slbd_batch *B, void **p, size_t bytes) {
+  *p = NULL;
+  if (mem_limit && B->bytes + bytes > mem_limit) return false;
+  if (hipMalloc(p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = NULL;
+    return false;
+  }
+  B->bytes += bytes;
+  return true;
+}
+
+/* Single steps from here on: their memory goes back. */
+static void drop_pairs(slbd_batch *B) {
+  void *ps[] = {B->place, B->wrows, B->tiles2};
+  for (size_t q = 0; q < sizeof ps / sizeof ps[0]; q++)
+    if (ps[q]) HIPCHECK(hipFree(ps[q]));
+  B->bytes -= B->pair_bytes;
+  B->pair_bytes = 0;
+  B->place = NULL; B->wrows = NULL; B->tiles2 = NULL;
+  B->pairs = 0;
+}
+
+template <typename P>
+static void must_alloc(slbd_batch *B, P **p, size_t bytes) {
+  void *v;
+  if (!try_alloc(B, &v, bytes)) {
+    if (B->pairs) {          /* what single steps need comes before the pairs' tables */
+      HIPCHECK(hipStreamSynchronize(B->stream));
+      drop_pairs(B);
+      invalidate_graphs(B);
+    }
+    if (!try_alloc(B, &v, bytes)) {
+      fprintf(stderr, "sunlightlb: out of device memory (%zu bytes for a batch)\n", bytes);
+      exit(EXIT_FAILURE);
+    }
+  }
+  *p = (P *)v;
+}
+
+/* memory that only the pairs need */
+template <typename P>
+static bool pair_alloc(slbd_batch *B, P **p, size_t bytes) {
+  void *v;
+  if (!try_alloc(B, &v, bytes)) return false;
+  B->pair_bytes += bytes;
+  *p = (P *)v;
+  return true;
+}
+
 static void build_tiles(slbd_batch *B) {
   const long per = (long)B->block * B->npt;
   long nt = 0;
@@ -579,8 +640,11 @@ static void build_tiles(slbd_batch *B) {
   long t = 0;
   for (int p = 0; p < B->nprob; p++)
     for (long s = 0; s < B->hprobs[p].N; s += per) { h[t].x = p; h[t].y = (int)s; t++; }
-  if (B->tiles) HIPCHECK(hipFree(B->tiles));
-  HIPCHECK(hipMalloc(&B->tiles, sizeof(int2) * (nt > 0 ? nt : 1)));
+  if (B->tiles) {
+    HIPCHECK(hipFree(B->tiles));
+    B->bytes -= sizeof(int2) * (B->ntiles > 0 ? B->ntiles : 1);
+  }
+  must_alloc(B, &B->tiles, sizeof(int2) * (nt > 0 ? nt : 1));
   HIPCHECK(hipMemcpy(B->tiles, h, sizeof(int2) * nt, hipMemcpyHostToDevice));
   free(h);
   B->ntiles = (int)nt;
@@ -711,19 +775,21 @@ static void plan_pairs(slbd_batch *B) {
   }
   B->ntiles2 = (int)n;
   B->thr2 = (pts + 63) & ~63;
-  HIPCHECK(hipMalloc(&B->tiles2, sizeof(int4) * (n > 0 ? n : 1)));
+  if (!pair_alloc(B, &B->tiles2, sizeof(int4) * (n > 0 ? n : 1))) {
+    drop_pairs(B);
+    free(h);
+    return;
+  }
   HIPCHECK(hipMemcpy(B->tiles2, h, sizeof(int4) * n, hipMemcpyHostToDevice));
   free(h);
   /* places of the boxes' boundary nodes, then the moving problems' rows */
   int *cnt, *hc = (int *)calloc(B->nbox, sizeof(int));
-  if (hipMalloc(&B->place, sizeof(int) * B->nnode_tab) != hipSuccess) {
-    (void)hipGetLastError();
-    B->place = NULL;
-    B->pairs = 0;
+  if (!pair_alloc(B, &B->place, sizeof(int) * B->nnode_tab) ||
+      !pair_alloc(B, &cnt, sizeof(int) * B->nbox)) {
+    drop_pairs(B);
     free(hc);
     return;
   }
-  HIPCHECK(hipMalloc(&cnt, sizeof(int) * B->nbox));
   HIPCHECK(hipMemsetAsync(cnt, 0, sizeof(int) * B->nbox, B->stream));
   long nrow = 0;
   for (int b = 0; b < B->nbox; b++) {
@@ -736,6 +802,8 @@ static void plan_pairs(slbd_batch *B) {
   HIPCHECK(hipMemcpyAsync(hc, cnt, sizeof(int) * B->nbox, hipMemcpyDeviceToHost, B->stream));
   HIPCHECK(hipStreamSynchronize(B->stream));
   HIPCHECK(hipFree(cnt));
+  B->bytes -= sizeof(int) * B->nbox;
+  B->pair_bytes -= sizeof(int) * B->nbox;
   for (int b = 0; b < B->nbox; b++)
     if (B->box[b].moving)
       for (int r = 0; r < B->box[b].nrhs; r++) {
@@ -743,10 +811,8 @@ static void plan_pairs(slbd_batch *B) {
         nrow += hc[b];
       }
   /* a batch that fills the memory without the rows runs single steps */
-  if (hipMalloc(&B->wrows, bts(B->prec) * 16 * (nrow > 0 ? nrow : 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    B->wrows = NULL;
-    B->pairs = 0;
+  if (!pair_alloc(B, &B->wrows, bts(B->prec) * 16 * (nrow > 0 ? nrow : 1))) {
+    drop_pairs(B);
     free(hc);
     return;
   }
@@ -792,18 +858,18 @@ extern "C" int slbd_batch_commit(slbd_batch *B) {
   B->npop_total = pops;
   B->hprobs = (BProb *)calloc(nprob, sizeof(BProb));
   B->box_first_prob = (int *)malloc(sizeof(int) * B->nbox);
-  HIPCHECK(hipMalloc(&B->pops[0], bts(B->prec) * pops));
-  HIPCHECK(hipMalloc(&B->pops[1], bts(B->prec) * pops));
+  must_alloc(B, &B->pops[0], bts(B->prec) * pops);
+  must_alloc(B, &B->pops[1], bts(B->prec) * pops);
   HIPCHECK(hipMemsetAsync(B->pops[0], 0, bts(B->prec) * pops, B->stream));
   HIPCHECK(hipMemsetAsync(B->pops[1], 0, bts(B->prec) * pops, B->stream));
-  HIPCHECK(hipMalloc(&B->flags, sizeof(uint16_t) * nodes));
-  HIPCHECK(hipMalloc(&B->objidx, sizeof(int32_t) * nodes));
+  must_alloc(B, &B->flags, sizeof(uint16_t) * nodes);
+  must_alloc(B, &B->objidx, sizeof(int32_t) * nodes);
   int32_t *dmask;
-  HIPCHECK(hipMalloc(&dmask, sizeof(int32_t) * nodes));
-  HIPCHECK(hipMalloc(&B->tab, sizeof(double) * SLBD_OBJ_STRIDE * (ntab > 0 ? ntab : 1)));
-  HIPCHECK(hipMalloc(&B->wtab, bts(B->prec) * WROW * (ntab > 0 ? ntab : 1)));
+  must_alloc(B, &dmask, sizeof(int32_t) * nodes);
+  must_alloc(B, &B->tab, sizeof(double) * SLBD_OBJ_STRIDE * (ntab > 0 ? ntab : 1));
+  must_alloc(B, &B->wtab, bts(B->prec) * WROW * (ntab > 0 ? ntab : 1));
   double *hw = (double *)calloc((size_t)WROW * (ntab > 0 ? ntab : 1), sizeof(double));
-  HIPCHECK(hipMalloc(&B->acc, sizeof(double) * 6 * (nacc > 0 ? nacc : 1)));
+  must_alloc(B, &B->acc, sizeof(double) * 6 * (nacc > 0 ? nacc : 1));
   HIPCHECK(hipMemsetAsync(B->acc, 0, sizeof(double) * 6 * (nacc > 0 ? nacc : 1), B->stream));
   B->hacc = (double *)calloc(6 * (size_t)(nacc > 0 ? nacc : 1), sizeof(double));
   if (!B->hacc) { fprintf(stderr, "sunlightlb: out of host memory\n"); exit(EXIT_FAILURE); }
@@ -865,13 +931,16 @@ extern "C" int slbd_batch_commit(slbd_batch *B) {
   free(hw);
   HIPCHECK(hipStreamSynchronize(B->stream));
   HIPCHECK(hipFree(dmask));
+  B->bytes -= sizeof(int32_t) * nodes;
+  /* what single steps need first: the pairs take what is left, or do without */
+  must_alloc(B, &B->probs, sizeof(BProb) * nprob);
+  build_tiles(B);
   plan_pairs(B);
-  HIPCHECK(hipMalloc(&B->probs, sizeof(BProb) * nprob));
   HIPCHECK(hipMemcpy(B->probs, B->hprobs, sizeof(BProb) * nprob, hipMemcpyHostToDevice));
   long tot = 0;
   for (int q = 0; q < nprob; q++) tot += B->hprobs[q].N;
   B->nnodes_total = tot;
-  build_tiles(B);
+  last_bytes = B->bytes;
   B->committed = 1;
   return 0;
 }

@@ -215,3 +215,57 @@ def test_every_addressing_mode_is_single_steps(dims, stokes, skip, bf, nt, mode,
         assert np.array_equal(ref.pops(), got.pops())
     ref.free()
     got.free()
+
+
+def limited_batch(limit, env, monkeypatch):
+    """A committed batch under a limit of device memory (0: none): its handle,
+    the bytes it holds, and the populations after 35 steps and 3 more at
+    another launch shape."""
+    monkeypatch.setenv("SLB_BATCH_STEP2", env)
+    lats = [build(d, 32, 1, 1, 0, 0) for d in ((33, 31, 29), (40, 24, 36))]
+    L = lats[0].L
+    L.slbd_batch_mem_limit.argtypes, L.slbd_batch_mem_limit.restype = [C.c_size_t], C.c_size_t
+    b = L.slb_batch_new(32)
+    for lat in lats:
+        n = len(lat.objects())
+        vel = np.random.default_rng(n).normal(0, 0.01, (3, n, 6))
+        L.slb_batch_add(b, lat.h, 3, vel.ctypes.data_as(C.POINTER(C.c_double)))
+        lat.free()
+    try:
+        L.slbd_batch_mem_limit(limit)
+        assert L.slb_batch_commit(b) == 0
+        held = L.slbd_batch_mem_limit(limit)
+        kernel = L.slb_batch_run_kernel(b).decode()
+        L.slb_batch_run(b, 35)
+        L.slb_batch_set_config(b, 64, 1, 0)      # four times the tiles
+        L.slb_batch_run(b, 3)
+    finally:
+        L.slbd_batch_mem_limit(0)
+    out = []
+    for q, n in enumerate((33 * 31 * 29, 40 * 24 * 36)):
+        a = np.zeros(15 * n)
+        L.slb_batch_get_pops(b, q, 2, a.ctypes.data_as(C.POINTER(C.c_double)))
+        out.append(a)
+    after = L.slb_batch_run_kernel(b).decode()
+    L.slb_batch_free(b)
+    return held, kernel, after, out
+
+
+def test_batch_without_memory_for_pairs_runs_single_steps(monkeypatch):
+    """The tables of single steps come before those of the pairs: whatever is
+    left for the latter, the batch runs, with the same results."""
+    single, k, _, ref = limited_batch(0, "0", monkeypatch)
+    pairs, k2, after, got = limited_batch(0, "1", monkeypatch)
+    assert (k, k2, after) == ("k_bstep", "k_bstep2", "k_bstep2") and pairs > single
+    assert all(np.array_equal(a, c) for a, c in zip(ref, got))
+    # from what single steps hold (and commit needs for the masks, and the tiles of
+    # the second shape) up to a byte too few
+    least = single + 4 * (33 * 31 * 29 + 40 * 24 * 36) + 40000
+    assert least < pairs
+    for limit in (least, (single + pairs) // 2, pairs - 1, pairs, pairs + 20000):
+        held, k, after, got = limited_batch(limit, "1", monkeypatch)
+        print(f"batch memory limit {limit}: holds {held}, {k}, {after}", flush=True)
+        assert held <= limit and k == ("k_bstep2" if limit >= pairs else "k_bstep")
+        # the second shape's tiles (18 kB more) take the pairs' memory where there is no other
+        assert after == ("k_bstep2" if limit >= pairs + 20000 else "k_bstep")
+        assert all(np.array_equal(a, c) for a, c in zip(ref, got))
