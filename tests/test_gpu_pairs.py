@@ -64,6 +64,64 @@ def test_run_is_single_steps(prec, dims, moving, stokes, skip, bf):
 
 
 @pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("dims,stokes,skip,bf", [
+    ((9, 32, 64), 0, 1, 2), ((9, 32, 64), 1, 0, 2), ((5, 8, 512), 1, 1, 0), ((4, 11, 331), 0, 0, 1),
+    ((1, 1, 7), 0, 0, 1), ((1, 40, 50), 0, 1, 2), ((3, 2, 1), 1, 1, 2), ((300, 4, 4), 0, 0, 1),
+])
+def test_pairs_with_walls_at_rest(prec, dims, stokes, skip, bf, monkeypatch):
+    """The shapes that test_run_is_single_steps runs with moving walls, which
+    take single steps, with walls at rest, in pairs: one plane, whole tiles with
+    a force per node, k tiles of unequal width, a long march."""
+    monkeypatch.setenv("SLB_STEP2", "1")
+    ref, got = (build(dims, prec, 0, stokes, skip, bf) for _ in range(2))
+    assert got.L.slb_run_kernel(got.h) == b"k_step2"
+    for n in (2, 7):
+        for _ in range(n):
+            ref.L.lbstep(ref.h)
+        got.L.slb_run(got.h, n)
+        assert np.array_equal(ref.pops(), got.pops())
+    ref.free()
+    got.free()
+
+
+@pytest.mark.parametrize("dims,mode", [((1, 6016, 6016), 3), ((1, 6000, 6001), 3), ((4, 3072, 3072), 2)])
+def test_pairs_on_buffers_over_4_gb(dims, mode, monkeypatch):
+    """FP64: one plane of 4.3 GB, whose byte offsets do not fit 32 bits, of whole
+    tiles and ragged; four planes of 1.1 GB.  Momentum and density of every node
+    after 4 steps, bit for bit."""
+    import sunlightlb_amd as s
+    monkeypatch.setenv("SLB_STEP2", "1")
+    n, out, d = dims[1], [], None
+    for pairs in (0, 1):
+        print(f"lattice {dims}, pairs {pairs}", flush=True)
+        lat = s.Lattice(*dims, precision=64)
+        L, h = lat.L, lat.h
+        L.slbd_step2_mode.argtypes = [C.c_long, C.c_long, C.c_int]
+        assert 15 * lat.N * 8 > 1 << 32
+        assert L.slbd_step2_mode(dims[1] * dims[2], lat.N, 64) == mode
+        lat.s.tau, lat.s.stokes_flow = 0.8, 0
+        for q in range(4):
+            L.insertcyl(h, b"x", 40.0, n * (0.12 + 0.25 * q), n * (0.98 - 0.27 * q))
+        L.zerobf(h)
+        lat.s.dpdx, lat.s.dpdy, lat.s.dpdz = 1e-5, 2e-5, -3e-5
+        if pairs:
+            assert L.slb_run_kernel(h) == b"k_step2"
+            L.slb_run(h, 4)
+        else:
+            for _ in range(4):
+                L.lbstep(h)
+        d = d or L.slbn_malloc(lat.N * 4 * 4)
+        L.slb_warm_moments(h, d, 4, 1.0)
+        a = np.empty(lat.N * 4, np.float32)
+        L.slbn_d2h(a.ctypes.data, d, a.nbytes)
+        out.append(a)
+        L.slb_destroy(h)
+    L.slbn_free(d)
+    last = out[0].reshape(-1, 4)[-64:]
+    assert np.all(last[:, 1] != 0.0) and np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("prec", [64, 32])
 @pytest.mark.parametrize("dims,nmom,axis,pads,moving", [
     ((9, 32, 64), 3, 0, 0.01, 0),
     ((7, 13, 131), 3, 1, 0.3, 0),     # remainders in j and k, more than one k tile
