@@ -289,3 +289,68 @@ def test_weight_gradient_in_a_captured_graph():
             d.free()
     for d in (dX, dG, dW):
         d.free()
+
+
+@pytest.mark.parametrize("C,N", [(16, 300001), (64, 40000), (8, 5000), (32, 7), (256, 3000), (4, 70000)])
+def test_bias_gradient_is_the_same_at_every_call(C, N):
+    """The blocks' sums in a fixed order: 8 calls bit for bit, added to what is
+    there; with atomics (no workspace) to rounding."""
+    L = lib()
+    rng = np.random.default_rng(C + N)
+    yb, y = bf_random(rng, (N, C))
+    gb, g = bf_random(rng, (N, C))
+    dY, dG, dP = Dev(host=yb), Dev(host=gb), Dev(N * C * 2)
+    was = rng.standard_normal(C).astype(np.float32)
+    ref = np.where(y > 0, g, 0.0).sum(0) + was
+    scale = np.abs(g).sum(0).max()
+    got = []
+    for _ in range(8):
+        db = Dev(host=was)
+        L.slbn_relu_bwd_bias(dY.p, dG.p, dP.p, C, N, db.p)
+        L.slbn_sync()
+        got.append(db.get(np.uint32, (C,)))
+        db.free()
+    for d in (dY, dG, dP):
+        d.free()
+    assert all(np.array_equal(a, got[0]) for a in got)
+    assert np.abs(got[0].view(np.float32) - ref).max() < 1e-5 * scale
+
+
+def test_bias_gradient_without_a_workspace(monkeypatch):
+    monkeypatch.setenv("SLBN_WGRAD_WS", "0")
+    L, N, C = lib(), 9000, 32
+    gb, g = bf_random(np.random.default_rng(8), (N, C))
+    dG, db = Dev(host=gb), Dev(C * 4)
+    L.slbn_bias_grad(dG.p, C, N, db.p)
+    L.slbn_sync()
+    assert np.abs(db.get(np.float32, (C,)) - g.sum(0)).max() < 1e-5 * np.abs(g).sum(0).max()
+    dG.free()
+    db.free()
+
+
+@pytest.mark.parametrize("dims", [(16, 24, 32), (16, 16, 40), (24, 16, 72)])
+def test_training_can_be_repeated(dims):
+    """Two networks of one seed trained on the same packs: the same weights, bit
+    for bit (rows that the LDS-staged, the blocked and the padded weight
+    gradients take)."""
+    import sunlightlb_amd as s
+    L, out = lib(), []
+    for _ in range(2):
+        net = L.slb_warm_new(3)
+        for q in range(3):
+            lat = s.Lattice(*dims, precision=32)
+            lat.s.tau, lat.s.stokes_flow = 0.75, 1
+            rng = np.random.default_rng(q)
+            for _ in range(4):
+                L.insertsph(lat.h, 3.0, *[float(rng.uniform(0, n)) for n in dims])
+            L.zerobf(lat.h)
+            L.addbf(lat.h, 1e-6, 0.0, 0.0)
+            L.slb_run(lat.h, 200)
+            L.slb_warm_add_sample(net, lat.h)
+            lat.free()
+        L.slb_warm_train(net, 40, 1e-3, 5, None)
+        w = np.empty(L.slb_warm_nparams(net), np.float32)
+        L.slb_warm_get_params(net, w.ctypes.data)
+        L.slb_warm_free(net)
+        out.append(w)
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
