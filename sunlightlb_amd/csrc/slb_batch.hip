@@ -669,8 +669,9 @@ static double block_us(int prec, int moving, int pts, int ci) {
 
 /* Whether a batch takes two steps per pass, and the tiles of every box (box: esi, esj, esk, right-hand sides, moving; tile: jt, kt,
  * ci), and the time of two steps in this way and as two single ones (us).  Tried
- * are tiles of at most `cap` threads and chunks of at most `len` planes; a CU
- * holds one block at a time.  Large tiles and long chunks do the least work, but
+ * are tiles of at most `cap` threads (of these the split of a plane that costs
+ * least, as slbd_step2_plan: FP64 512 boxes x 6 10.6 ms per step, 10.9 by block_us)
+ * and chunks of at most `len` planes; a CU holds one block at a time.  Large tiles and long chunks do the least work, but
  * few problems then leave most CUs idle: one box of 64^3, FP32, us per step: 20
  * blocks (13 x 64 x 16) 21.4, 256 (8 x 64 x 2) 6.3, single steps 7.6; one right-hand
  * side of 6 of 64^3 35.1/19.3 (single / this), 2 x 2 of 256 x 256 x 4 25.3/15.2 (62 in
@@ -700,7 +701,7 @@ extern "C" int slbd_bstep2_plan(int nbox, const int *box, int prec, int *tile, d
         for (int jq = 1; jq <= q[1] && (jq + 2) * (k + 2) <= caps[c]; jq++) {
           const int njt = (q[1] + jq - 1) / jq, j = (q[1] + njt - 1) / njt;
           const double cost = (1.0 + 16.0 / k) * njt * nkt *
-                              block_us(prec, q[4], (j + 2) * (k + 2), 1 << 20);
+                              ((double)(j + 2) * (k + 2) + (double)j * k + 1000.0);
           if (jt == 0 || cost < bc) { bc = cost; jt = j; kt = k; }
         }
       }
