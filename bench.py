@@ -511,8 +511,8 @@ def batch_run(L, args, prec, boxes, u0, tau, tune):
 def batch_workload(L, args, u0=1e-3, tau=1.0):
     """512 independent periodic boxes, each with 6 right-hand sides (unit
     translation and rotation of sphere 0, the other spheres fixed), stepped
-    together: one launch per step over all problems, autotuned launch shape,
-    HIP-graph replay.  Reports throughput and the 6x6 resistance matrices of
+    together: one launch per one or two steps over all problems (single steps of
+    the autotuned launch shape), HIP-graph replay.  Reports throughput and the 6x6 resistance matrices of
     sphere 0 after measure(); an FP32 batch is repeated in FP64 (same launch
     shape class, not timed against it) and the matrices are compared."""
     import numpy as np

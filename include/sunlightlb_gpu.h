@@ -73,12 +73,12 @@ int slb_run_to_residual_aa(LBSys lb, double tol, int interval, int maxsteps, int
 double slb_time_steps(LBSys lb, int nsteps);
 
 /* Name of the kernel that the lattice's single fused steps launch (lbstep, and
- * runs with moving walls; other runs take their steps in pairs, k_step2),
- * fixed when the lattice is made from its shape and precision: "k_step_lds" (rows of 64,
+ * the runs that do not take their steps in pairs, slb_run_kernel), fixed when
+ * the lattice is made from its shape and precision: "k_step_lds" (rows of 64,
  * 128, 256 or 512 nodes, k pulls staged in LDS), "k_step_ldsr" (other rows
  * of up to 512 nodes, where staging measured faster) or "k_step".  All of
- * them give bit-identical results; SLB_STEP_LDS=0 selects k_step for every
- * step, SLB_STEP2=0 keeps runs to single steps. */
+ * them, and k_step2, give bit-identical results; SLB_STEP_LDS=0 selects k_step
+ * for every step, SLB_STEP2=0 keeps runs to single steps. */
 const char *slb_step_kernel(LBSys lb);
 
 /* Name of the kernel that slb_run's steps launch as the lattice stands now
@@ -190,8 +190,10 @@ int  slb_batch_add(SLBBatch b, LBSys lb, int nrhs, const double *objvel);
 /* Allocate the device arenas and the tile schedule; no more boxes after. */
 int  slb_batch_commit(SLBBatch b);
 
-/* Choose block size, nodes per thread and persistent grid size by timing
- * candidate shapes on this batch (before its first step; the state is reset
+/* Choose block size, nodes per thread and persistent grid size of the single
+ * steps (k_bstep: every step of a batch on single steps, else an odd last one and
+ * measure; two steps per pass have their own tiles) by timing candidate shapes on
+ * this batch (before its first step; the state is reset
  * to rest afterwards).  With cache_path, a shape class already in the file is
  * reused without timing, and new results are appended.  Returns 1 on a cache
  * hit, 0 after timing, -1 on error. */

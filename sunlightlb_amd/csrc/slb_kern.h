@@ -116,7 +116,7 @@ struct Geom {
                     XCD, T >= 2 tiles of T x T rows per XCD */
   int nt_store;  /* step kernel: non-temporal population stores */
   int nt_load;   /* step kernel: non-temporal population loads */
-  int step_tpb;  /* step kernel: threads per block (256 or 512) */
+  int step_tpb;  /* step kernel: threads per block (128, 256 or 512) */
   int mp_xcd;    /* moment-propagation kernel block order (as xcd_map: 0 or 1) */
 };
 

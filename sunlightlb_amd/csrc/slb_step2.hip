@@ -19,7 +19,8 @@
  * Bound by HBM and its latency at 256^3: FP32 2.36 GB for two steps (1.17x
  * one read and one write), 80% of the copy rate, the VALU busy 40% of the
  * time; FP64 4.82 GB, 98%, 29%.  Measured, us per step, one
- * step at a time / this kernel: FP32 256^3 356.6/224.0, 512^3 2957/1852,
+ * step at a time / this kernel: FP32 256^3 356.6/224.0 (252 on the slowest
+ * card), 512^3 2957/1852,
  * 160^3 94.4/58.8, 96^3 20.7/12.6, 64^3 6.97/6.05; FP64 256^3 735/401,
  * 128^3 92.9/54.7, 32^3 5.69/3.87.
  *
@@ -32,9 +33,10 @@
  * for its loads and stores (239 us).  The LDS is double buffered: one barrier
  * per plane.  Every node runs the arithmetic of k_step (bounce-back,
  * collide_node): bit-identical results.  Walls are at rest: with the wall
- * terms of moving objects, their FP64 velocity loads and the registers these
- * take, the pair was slower than two steps (FP64 128^3 116 against 102 us per
- * step, FP32 256^3 1323 against 388).
+ * terms of moving objects looked up link by link, their FP64 velocity loads and
+ * the registers these take, the pair was slower than two steps (FP64 128^3 116
+ * against 102 us per step, FP32 256^3 1323 against 388); rows of precomputed
+ * terms, as k_bstep2 has them, were not tried here.
  */
 #include "slb_dev.h"
 #include "slb_kern.h"
