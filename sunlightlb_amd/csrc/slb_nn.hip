@@ -1197,9 +1197,14 @@ struct WgSpace {
 static WgSpace wg_space[WG_STREAMS];
 static std::mutex wg_mutex;
 
+/* (asked of the null stream, HIP answers with an error while another one is
+ * captured) */
 static bool nn_capturing(void) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  HIPCHECK(hipStreamIsCapturing(nn_stream, &st));
+  if (hipStreamIsCapturing(nn_stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
   return st != hipStreamCaptureStatusNone;
 }
 
